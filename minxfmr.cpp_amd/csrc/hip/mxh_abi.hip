@@ -75,7 +75,7 @@ int gemm_q_f16_body(const char* who, int type, const float* a, int64_t m, const 
                                     (int)k / 32, r.rscale, (int)m, g_ctx.stream))
         return set_error(rc, "%s: conversion launch", who);
     if (int rc = gemm_q_f16_run(type, r.a_hi, r.a_lo, (int)k, r.s_hi, r.s_lo, (int)k / 32, r.rscale, w, out, (int)n,
-                                nullptr, (int)m, (int)n, (int)k, form, nullptr, 0, g_ctx.stream))
+                                nullptr, (int)m, (int)n, (int)k, form, g_ctx.stream))
         return set_error(rc, "%s: launch", who);
     return check_hip(hipGetLastError(), who);
 }
@@ -84,7 +84,7 @@ int gemm_q_f16_check(const char* who, int type, const float* a, int64_t m, const
                      float* out) {
     if (!a || !w || !out) return set_error(MXH_ERR_ARG, "%s: null pointer", who);
     if (m <= 0 || n <= 0 || k <= 0 || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX ||
-        !gemm_q_f16_supported(type, (int)k))
+        storage_type(type) == MXH_Q6_K || !gemm_q_f16_supported(type, (int)k))
         return set_error(MXH_ERR_ARG, "%s: bad shape %lldx%lldx%lld for type %d", who, (long long)m, (long long)n,
                          (long long)k, type);
     if (((uintptr_t)w & 15) || ((uintptr_t)a & 15))
@@ -185,6 +185,7 @@ int mxh_init(int device) {
     void* sp = nullptr;
     if (int rc = check_hip(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)")) return rc;
     g_scratch_ptr[device] = sp;
+    if (int rc = gemm_workspace_init()) return rc;
     if (int rc = check_hip(hipStreamCreateWithFlags(&g_ctx.stream, hipStreamNonBlocking), "hipStreamCreate")) return rc;
     if (int rc = check_hip(hipEventCreate(&g_ctx.ev0), "hipEventCreate")) return rc;
     if (int rc = check_hip(hipEventCreate(&g_ctx.ev1), "hipEventCreate")) return rc;
