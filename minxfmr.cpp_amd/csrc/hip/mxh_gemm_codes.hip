@@ -24,9 +24,13 @@
 // Shape of the kernel.  8 waves, one workgroup per CU: WM along the
 // activation rows x WN = 8 / WM along the weight rows, each wave 32 MI x
 // 32 NJ outputs of v_mfma_f32_32x32x16_f16.  A K step is 64 elements.  The
-// raw weight bytes and the activations go straight into LDS
-// (global_load_lds_dwordx4), NST stages in flight, one barrier per step;
-// every wave decodes the weight rows it multiplies itself, from LDS.
+// activations of a step and the raw weight bytes of a granule (two or four
+// steps) go straight into LDS (global_load_lds_dwordx4), one barrier per step;
+// every wave decodes the weight rows it multiplies itself, from LDS.  The
+// granule is there for the memory pipe: a load whose lanes read 16 bytes of 64
+// different rows takes about 60 ns of a CU on a full chip, a quarter of that
+// when four lanes share 64 consecutive bytes (codes loaded a step at a time:
+// 2241 against 2156 ns per 128 x 256 step, 907 against 675 per 32 x 256).
 //
 // What bounds it.  Per 128 x 256 x 64 step a SIMD has 2048 cycles of matrix
 // work (two products) and about 130 VALU instructions per wave (1040 cycles):
@@ -39,9 +43,10 @@
 //
 // Measured (one MI355X, this kernel against a 128-row-tile kernel for Q4_K
 // and an unpipelined one for the other types): Q4_K 512 x 24576 x 4096
-// 285 -> 250 us (412 TFLOP/s, 824 issued; a bf16 library product of 8192^3
-// reaches 1200), Q5_K 129 x 4096 x 14336 665 -> 74 us, Q8_0
-// 31 x 6144 x 1024 33 -> 17 us with the conversion of the rows.
+// 283 -> 238 us, 512 x 4096 x 12288 at 104 us (498 TFLOP/s, 996 issued; a bf16
+// library product of 8192^3 reaches 1200), Q5_K 129 x 4096 x 14336
+// 665 -> 72 us, Q8_0 31 x 6144 x 1024 33 -> 16 us with the conversion of the
+// rows.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -131,22 +136,18 @@ __device__ __forceinline__ f16x8 pack8(uint32_t a, uint32_t b, uint32_t c, uint3
 }
 
 // ---- weight formats --------------------------------------------------------
-// kQ 16-byte code pieces per row and step, kH 16-byte header pieces per row
-// and 256-element block; q_off / h_off: their byte offsets in a row of nblk
-// 256-element blocks, for step c (64 elements) and block b.  The offsets are
-// the same for every row and 32-bit, so they are scalar arithmetic (the tiled
-// orders are those of mxh_types.h).
-// kQL: dwords of codes a lane reads per weight row and step; slice_chunk: the
-// activation chunk (aoff) of slice sl of half-step h; kPair: a half-step is
-// a whole 32-element block with its own d.
+// The codes of a row arrive in granules of kGR steps (64 elements each): kNT
+// runs of kNC 16-byte pieces that lie side by side in the row, so that a load
+// instruction reads 16 kNC consecutive bytes per row.  Piece p of step s of a
+// granule is piece chunk(s, p) of run type(p).  kH 16-byte header pieces per
+// row and 256-element block.  q_off / h_off: the runs' and headers' byte
+// offsets in a row of nblk 256-element blocks; they are the same for every row
+// and 32-bit, so they are scalar arithmetic (the tiled orders are those of
+// mxh_types.h).  kQL: dwords of codes a lane reads per weight row and step;
+// slice_chunk: the activation chunk (aoff) of slice sl of half-step h; kPair: a
+// half-step is a whole 32-element block with its own d.
 template <int F>
 struct Fmt;
-
-struct FmtK {  // a 64-element group: low then high nibbles of 16 code bytes per lane half
-    static constexpr bool kMin = true, kSplitW = false, kRuns = false, kPair = false;
-    static constexpr int kQ = 2, kQL = 4;
-    static __host__ __device__ constexpr int slice_chunk(int half, int sl) { return half + 2 * sl; }
-};
 
 // blocks in tile j of tiles of T blocks
 template <int T>
@@ -155,54 +156,67 @@ __device__ __forceinline__ uint32_t tile_blocks(uint32_t j, uint32_t nblk) {
     return left < T ? left : T;
 }
 
-template <bool TILED>
-struct FmtQ4K : FmtK {
+struct FmtK {  // a 64-element group: low then high nibbles of 16 code bytes per lane half
+    static constexpr bool kMin = true, kSplitW = false, kRuns = false, kPair = false;
+    static constexpr int kQL = 4, kGR = 4;
+    static __host__ __device__ constexpr int slice_chunk(int half, int sl) { return half + 2 * sl; }
+};
+struct FmtKRow : FmtK {  // a block's 128 code bytes side by side
+    static constexpr int kNT = 1, kNC = 8;
+    static __device__ __forceinline__ int type(int) { return 0; }
+    static __device__ __forceinline__ int chunk(int s, int p) { return 2 * s + p; }
+};
+
+template <>
+struct Fmt<GF_Q4K> : FmtKRow {
     static constexpr int kType = MXH_Q4_K, kH = 1;
-    static __device__ __forceinline__ uint32_t q_off(uint32_t c, uint32_t p, uint32_t nblk) {
-        if constexpr (TILED) {
-            const uint32_t j = c >> 6, t = tile_blocks<16>(j, nblk);
-            return j * 2304 + 16 * (t + (c & 63) + 4 * t * p);
-        }
-        return (c >> 2) * 144 + 16 + 32 * (c & 3) + 16 * p;
+    static __device__ __forceinline__ uint32_t q_off(uint32_t b, uint32_t, uint32_t) { return b * 144 + 16; }
+    static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t, uint32_t) { return b * 144; }
+};
+template <>
+struct Fmt<GF_Q4KT> : FmtK {
+    static constexpr int kType = MXH_Q4_K, kH = 1, kNT = 2, kNC = 4;
+    static __device__ __forceinline__ int type(int p) { return p; }
+    static __device__ __forceinline__ int chunk(int s, int) { return s; }
+    static __device__ __forceinline__ uint32_t q_off(uint32_t b, uint32_t t, uint32_t nblk) {
+        const uint32_t j = b >> 4, nb = tile_blocks<16>(j, nblk);
+        return j * 2304 + 16 * (nb + 4 * (b & 15) + 4 * nb * t);
     }
     static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t, uint32_t) {
-        return TILED ? (b >> 4) * 2304 + 16 * (b & 15) : b * 144;
+        return (b >> 4) * 2304 + 16 * (b & 15);
     }
 };
-template <> struct Fmt<GF_Q4K> : FmtQ4K<false> {};
-template <> struct Fmt<GF_Q4KT> : FmtQ4K<true> {};
-
-template <bool TILED>
-struct FmtQ5K : FmtK {
+template <>
+struct Fmt<GF_Q5K> : FmtKRow {
     static constexpr int kType = MXH_Q5_K, kH = 3;
-    static __device__ __forceinline__ uint32_t q_off(uint32_t c, uint32_t p, uint32_t nblk) {
-        if constexpr (TILED) {  // 32-element chunks 2 c, 2 c + 1: adjacent pieces
-            const uint32_t j = c >> 5;
-            return j * 1408 + 16 * (3 * tile_blocks<8>(j, nblk) + 2 * (c & 31) + p);
-        }
-        return (c >> 2) * 176 + 48 + 32 * (c & 3) + 16 * p;
+    static __device__ __forceinline__ uint32_t q_off(uint32_t b, uint32_t, uint32_t) { return b * 176 + 48; }
+    static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t p, uint32_t) { return b * 176 + 16 * p; }
+};
+template <>
+struct Fmt<GF_Q5KT> : FmtKRow {
+    static constexpr int kType = MXH_Q5_K, kH = 3;
+    static __device__ __forceinline__ uint32_t q_off(uint32_t b, uint32_t, uint32_t nblk) {
+        const uint32_t j = b >> 3;
+        return j * 1408 + 16 * (3 * tile_blocks<8>(j, nblk) + 8 * (b & 7));
     }
     static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t p, uint32_t nblk) {
-        if constexpr (TILED) {
-            const uint32_t j = b >> 3, l = b & 7;
-            return j * 1408 + (p == 0 ? 16 * l : 16 * tile_blocks<8>(j, nblk) + 32 * l + 16 * (p - 1));
-        }
-        return b * 176 + 16 * p;
+        const uint32_t j = b >> 3, l = b & 7;
+        return j * 1408 + (p == 0 ? 16 * l : 16 * tile_blocks<8>(j, nblk) + 32 * l + 16 * (p - 1));
     }
 };
-template <> struct Fmt<GF_Q5K> : FmtQ5K<false> {};
-template <> struct Fmt<GF_Q5KT> : FmtQ5K<true> {};
 
-// a step is two 32-element blocks: pieces (first, last 16 codes) of each; the
-// header is the eight fp16 d of 256 elements
+// a step is two 32-element blocks, pieces (first, last 16 codes) of each; a
+// granule is four of them; the header is the eight fp16 d of 256 elements
 template <>
 struct Fmt<GF_Q80T> {
-    static constexpr int kType = MXH_Q8_0, kQ = 4, kH = 1, kQL = 8;
+    static constexpr int kType = MXH_Q8_0, kH = 1, kQL = 8, kGR = 2, kNT = 2, kNC = 4;
     static constexpr bool kMin = false, kSplitW = false, kRuns = false, kPair = true;
     static __host__ __device__ constexpr int slice_chunk(int half, int sl) { return 2 * half + sl; }
-    static __device__ __forceinline__ uint32_t q_off(uint32_t c, uint32_t p, uint32_t nblk) {
-        const uint32_t j = c >> 5, l = 2 * (c & 31) + (p >> 1);
-        return j * 2176 + 16 * (l + (p & 1) * tile_blocks<64>(j, 8 * nblk));
+    static __device__ __forceinline__ int type(int p) { return p & 1; }
+    static __device__ __forceinline__ int chunk(int s, int p) { return 2 * s + (p >> 1); }
+    static __device__ __forceinline__ uint32_t q_off(uint32_t gr, uint32_t t, uint32_t nblk) {
+        const uint32_t j = gr >> 4;
+        return j * 2176 + 16 * (4 * (gr & 15) + t * tile_blocks<64>(j, 8 * nblk));
     }
     static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t, uint32_t nblk) {
         const uint32_t j = b >> 3;
@@ -214,12 +228,14 @@ struct Fmt<GF_Q80T> {
 // (kRuns: 32 apart), so the activations are staged in that order
 template <>
 struct Fmt<GF_Q6KT> {
-    static constexpr int kType = MXH_Q6_K, kQ = 3, kH = 1, kQL = 6;
+    static constexpr int kType = MXH_Q6_K, kH = 1, kQL = 6, kGR = 2, kNT = 3, kNC = 2;
     static constexpr bool kMin = false, kSplitW = true, kRuns = true, kPair = false;
     static __host__ __device__ constexpr int slice_chunk(int half, int sl) { return 2 * half + sl; }
-    static __device__ __forceinline__ uint32_t q_off(uint32_t c, uint32_t p, uint32_t nblk) {
-        const uint32_t j = c >> 6;
-        return j * 3360 + 16 * (4 * tile_blocks<16>(j, nblk) * p + (c & 63));
+    static __device__ __forceinline__ int type(int p) { return p; }
+    static __device__ __forceinline__ int chunk(int s, int) { return s; }
+    static __device__ __forceinline__ uint32_t q_off(uint32_t gr, uint32_t t, uint32_t nblk) {
+        const uint32_t j = gr >> 5;
+        return j * 3360 + 16 * (4 * tile_blocks<16>(j, nblk) * t + 2 * (gr & 31));
     }
     static __device__ __forceinline__ uint32_t h_off(uint32_t b, uint32_t, uint32_t nblk) {
         const uint32_t j = b >> 4;
@@ -233,29 +249,38 @@ struct Fmt<GF_Q6KT> {
 };
 
 // ---- geometry ----------------------------------------------------------------
+// Activations are staged per step, NST slots; codes per granule and headers
+// (with the sub-block sums) per block, two slots each.  Slots are refilled at
+// the end of a step: the activations of step t + NST at the end of step t,
+// the next granule at the end of its predecessor's first step.
 template <int F, int WM, int MI, int NJ, int NST>
 struct Geo {
     using FM = Fmt<F>;
     static constexpr int WN = 8 / WM, BM = 32 * MI * WM, BN = 32 * NJ * WN;
-    static constexpr int kA = BM * 256;                    // activation bytes of a stage (hi, lo)
-    static constexpr int kAL = BM / 32;                    // direct loads per wave: activations,
-    static constexpr int kWL = (FM::kQ * BN + 511) / 512;  // code pieces,
+    static constexpr int kA = BM * 256;                   // activation bytes of a stage (hi, lo)
+    static constexpr int kAL = BM / 32;                   // direct loads per wave: activations of a stage,
+    static constexpr int kWN = FM::kNT * FM::kNC * BN;    // (pieces of a granule)
+    static constexpr int kWL = (kWN + 511) / 512;         // codes of a granule,
     static constexpr int kHN = FM::kH * BN + (FM::kMin ? 2 * BM : 0);
-    static constexpr int kHL = (kHN + 511) / 512;  // and, every fourth step, headers and sub-block sums
-    static constexpr int kDL = FM::kSplitW ? 1 : 0;  // 4-byte loads of d (Q6_K)
-    static constexpr int kStage = kA + FM::kQ * BN * 16;
-    static constexpr int kHdr = kHN * 16 + kDL * 2048;
-    static constexpr size_t kLds = (size_t)NST * kStage + 2 * (size_t)kHdr;
-    static_assert(NST >= 2 && NST <= 5, "two header slots serve at most five stages");
+    static constexpr int kHL = (kHN + 511) / 512;         // headers and sub-block sums of a block,
+    static constexpr int kDL = FM::kSplitW ? 1 : 0;       // 4-byte loads of d (Q6_K)
+    static constexpr int kW = kWN * 16, kHdr = kHN * 16 + kDL * 2048;
+    static constexpr size_t kLds = (size_t)NST * kA + 2 * (size_t)kW + 2 * (size_t)kHdr;
+    // codes before or after the activations of the same refill: before where
+    // the wait for the activations that follow must cover them
+    static constexpr bool kWFirst = FM::kGR == 2 || NST > 2;
+    static_assert(NST >= 2 && NST <= (FM::kGR == 2 ? 2 : 4), "a granule arrives before its first step");
     static_assert(kLds <= 160 * 1024, "LDS of a CU");
     static_assert(kHN % 64 == 0 && BN % 64 == 0 && BM % 32 == 0, "a wave's pieces are of one kind");
-    // direct loads issued for stage `st` (st mod 4 given)
-    static constexpr int loads(int st) { return kAL + kWL + ((st & 3) == 0 ? kHL + kDL : 0); }
-    // loads in flight behind stage t when it is awaited: those of the stages
-    // up to t + NST - 3 (t + NST - 2 is issued after the wait)
+    // direct loads of codes and headers issued at the end of step s (s mod 4 counts)
+    static constexpr int wloads(int s) {
+        return s % FM::kGR == 0 ? kWL + ((s + FM::kGR) % 4 == 0 ? kHL + kDL : 0) : 0;
+    }
+    // loads issued after the activations of step t + 1 and in flight when they
+    // are awaited at the end of step t
     static constexpr int ahead(int t) {
-        int n = 0;
-        for (int s = t + 1; s <= t + NST - 3; ++s) n += loads(s);
+        int n = kWFirst ? 0 : wloads(t + 1 - NST + 4);
+        for (int s = t + 2 - NST; s <= t - 1; ++s) n += kAL + wloads(s + 4);
         return n;
     }
 };
@@ -264,6 +289,10 @@ struct Geo {
 // operand reads: 8 consecutive rows take 8 different chunk slots)
 __device__ __forceinline__ int a_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
+// XOR of the piece index of weight row `row` in a run of NC pieces
+template <int NC>
+__device__ __forceinline__ int w_swz(int row) { return (row / (16 / NC)) & (NC - 1); }
+
 template <int F, int WM, int MI, int NJ, int NST>
 __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     using G = Geo<F, WM, MI, NJ, NST>;
@@ -271,7 +300,8 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     constexpr int BM = G::BM, BN = G::BN, WN = G::WN;
     extern __shared__ __align__(16) uint8_t smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-    const uint8_t* hdrs = smem + (size_t)NST * G::kStage;
+    const uint8_t* codes = smem + (size_t)NST * G::kA;
+    const uint8_t* hdrs = codes + 2 * (size_t)G::kW;
 
     // work item: split z, weight tile x, activation tile y, y fastest, dealt so
     // that XCD q (workgroup ids q, q + 8, ...) takes a contiguous range: the
@@ -303,14 +333,18 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     }
     const uint8_t* wrow0 = a.w + (size_t)n0 * rb;
     const uint64_t wbase = scalar_addr(wrow0);
+    // piece slot (type, row, c) holds the row's piece c ^ w_swz(row) of the run:
+    // a fixed piece of 16 consecutive rows takes 16 different bank groups
     uint32_t voff_w[G::kWL];
-    int piece[G::kWL], wslot[G::kWL];
+    int wtype[G::kWL], wslot[G::kWL];
 #pragma unroll
     for (int u = 0; u < G::kWL; ++u) {
-        const int s = (u * 512 + wave * 64) % (FM::kQ * BN);  // padding waves repeat real pieces (same bytes, same place)
+        const int s = (u * 512 + wave * 64) % G::kWN;  // padding waves repeat real pieces (same bytes, same place)
         wslot[u] = s;
-        piece[u] = s / BN;
-        voff_w[u] = (uint32_t)(min(n0 + s % BN + lane, a.n - 1) - n0) * (uint32_t)rb;
+        wtype[u] = s / (BN * FM::kNC);
+        const int i = s % (BN * FM::kNC) + lane, row = i / FM::kNC;
+        const int c = (i % FM::kNC) ^ w_swz<FM::kNC>(row);
+        voff_w[u] = (uint32_t)(min(n0 + row, a.n - 1) - n0) * (uint32_t)rb + 16u * (uint32_t)c;
     }
     const uint32_t voff_d =
         (uint32_t)(min(n0 + (wave * 64) % BN + lane, a.n - 1) - n0) * (uint32_t)rb;  // (waves past BN / 64 repeat rows)
@@ -335,31 +369,32 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
 #pragma unroll
     for (int u = 0; u < G::kAL; ++u)
         abase[u] = scalar_addr(((wave * G::kAL + u) / (BM / 8) ? a.a_lo : a.a_hi) + (size_t)m0 * a.lda);
-    // issue the loads of stage st (past the end: the last stage again, never
-    // read) into LDS stage slot `slot`; a stage that starts a 256-element
-    // block brings that block's headers and sums first
-    auto issue = [&](int st, int slot, bool head) __attribute__((always_inline)) {
-        const int s = min(st, steps - 1), c = 4 * b0 + s;
-        const uint32_t base = lds0 + (uint32_t)slot * G::kStage;
-        if (head) {  // st mod 4 == 0, known at every call
-            const int b = c >> 2;
-            const uint32_t hb = lds0 + NST * G::kStage + (uint32_t)((st >> 2) & 1) * G::kHdr;
+    // (past the end the last step's, granule's or block's bytes again, never read)
+    auto issue_a = [&](int st, int slot) __attribute__((always_inline)) {
+        const int c = 4 * b0 + min(st, steps - 1);
+        const int e = FM::kRuns ? 256 * (c >> 2) + 128 * ((c >> 1) & 1) + 16 * (c & 1) : 64 * c;
+#pragma unroll
+        for (int u = 0; u < G::kAL; ++u)
+            g2l_s(abase[u] + 2 * (uint32_t)e, voff_a[u], lds0 + (uint32_t)slot * G::kA + (wave * G::kAL + u) * 1024);
+    };
+    // the granule that starts at step st, with its block's headers if the block does
+    auto issue_w = [&](int st, bool head) __attribute__((always_inline)) {
+        const int c = 4 * b0 + min(st, steps - FM::kGR);
+        const uint32_t gr = (uint32_t)c / FM::kGR, b = (uint32_t)c >> 2;
+        if (head) {
+            const uint32_t hb = lds0 + NST * G::kA + 2 * G::kW + (uint32_t)((st >> 2) & 1) * G::kHdr;
 #pragma unroll
             for (int u = 0; u < G::kHL; ++u) {
                 uint32_t off = FM::h_off(b, hpiece[u], nblk);
                 // (arithmetic, not a branch: the step stays one block of code)
-                if constexpr (FM::kMin) off += (16u * (uint32_t)b - off) * is_sum[u];
+                if constexpr (FM::kMin) off += (16u * b - off) * is_sum[u];
                 g2l_v(hptr[u] + off, hb + hslot[u] * 16);
             }
             if constexpr (G::kDL) g2l4_s(wbase + FM::d_off(b, nblk), voff_d, hb + G::kHN * 16 + wave * 256);
         }
-        const int e = FM::kRuns ? 256 * (c >> 2) + 128 * ((c >> 1) & 1) + 16 * (c & 1) : 64 * c;
+        const uint32_t wb = lds0 + NST * G::kA + (uint32_t)((st / FM::kGR) & 1) * G::kW;
 #pragma unroll
-        for (int u = 0; u < G::kAL; ++u)
-            g2l_s(abase[u] + 2 * (uint32_t)e, voff_a[u], base + (wave * G::kAL + u) * 1024);
-#pragma unroll
-        for (int u = 0; u < G::kWL; ++u)
-            g2l_s(wbase + FM::q_off(c, piece[u], nblk), voff_w[u], base + G::kA + wslot[u] * 16);
+        for (int u = 0; u < G::kWL; ++u) g2l_s(wbase + FM::q_off(gr, wtype[u], nblk), voff_w[u], wb + wslot[u] * 16);
     };
 
     f32x16 acc[MI][NJ], P[MI][NJ];
@@ -384,9 +419,11 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
 
     // The step is software-pipelined in four regions of one 16-element product
     // slice each: while a slice multiplies, the next slice's activations are
-    // read from LDS and the next half-step's codes are decoded, and the next
-    // stage is awaited in the middle of the step, so that no wave waits for
-    // LDS, or for the others, with its matrix core idle.
+    // read from LDS and the next half-step's codes are decoded.  A stage's slot
+    // is refilled as soon as every wave has read its last operands (before
+    // the step's last slice), so NST - 1 stages are always in flight: with
+    // one fewer (refilled in the middle of the next step) a step could not be
+    // shorter than a stage's load latency, 1.1 - 1.6 us on a full chip.
     f16x8 A[2][2 * MI];           // activation operands (hi, lo per row block): this slice, the next
     uint32_t q[NJ][FM::kQL];      // raw codes of the step
     f16x8 W[2][2][NJ];            // decoded codes: half-step, slice
@@ -424,19 +461,25 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
             }
         }
     };
-    auto read_q = [&](const uint8_t* wq) __attribute__((always_inline)) {
+    // the raw codes of step t (st: t modulo the granule)
+    auto read_q = [&](int t, auto sc) __attribute__((always_inline)) {
+        constexpr int st = decltype(sc)::value % FM::kGR;
+        const uint8_t* wq = codes + (size_t)((t / FM::kGR) & 1) * G::kW;
+        auto piece = [&](int j, int p) {
+            return wq + (FM::type(p) * (BN * FM::kNC) + col[j] * FM::kNC + (FM::chunk(st, p) ^ w_swz<FM::kNC>(col[j]))) * 16;
+        };
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             if constexpr (F == GF_Q6KT) {
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
-                    const uint2 v = *reinterpret_cast<const uint2*>(wq + (p * BN + col[j]) * 16 + 8 * hh);
+                    const uint2 v = *reinterpret_cast<const uint2*>(piece(j, p) + 8 * hh);
                     q[j][2 * p] = v.x, q[j][2 * p + 1] = v.y;
                 }
             } else {
 #pragma unroll
-                for (int p = 0; p < FM::kQ / 2; ++p) {
-                    const uint4 v = *reinterpret_cast<const uint4*>(wq + ((2 * p + hh) * BN + col[j]) * 16);
+                for (int p = 0; p < FM::kQL / 4; ++p) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(piece(j, 2 * p + hh));
                     q[j][4 * p] = v.x, q[j][4 * p + 1] = v.y, q[j][4 * p + 2] = v.z, q[j][4 * p + 3] = v.w;
                 }
             }
@@ -591,34 +634,37 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     auto step = [&](int t, auto gc) __attribute__((always_inline)) {
         constexpr int g = decltype(gc)::value;
         using GN = std::integral_constant<int, (g + 1) & 3>;
-        const uint8_t* stg = smem + (size_t)slot * G::kStage;
+        const uint8_t* stg = smem + (size_t)slot * G::kA;
         const int nslot = slot == NST - 1 ? 0 : slot + 1;
-        const uint8_t* nstg = smem + (size_t)nslot * G::kStage;
+        const uint8_t* nstg = smem + (size_t)nslot * G::kA;
         // a: slice (0, 0)
         read_a(stg, 0, 1, 1);
         MXH_CODES_FENCE();
         multiply(0, 0, 0, g == 0 || FM::kPair);
         if constexpr (FM::kMin && g == 1) min_terms(t);
         MXH_CODES_FENCE();
-        // b: slice (0, 1); stage t + 1 arrives, stage t + NST - 1 departs (its
-        // slot was read in step t - 1)
+        // b: slice (0, 1)
         read_a(stg, 1, 0, 0);
-        wait_vm<G::ahead(g + 1)>();
-        lds_barrier();
-        issue(t + NST - 1, slot == 0 ? NST - 1 : slot - 1, (g + NST - 1) % 4 == 0);
         MXH_CODES_FENCE();
         multiply(0, 1, 1, false);
         decode(gc, C1{});
         if constexpr (FM::kPair) fold(d2[0]);
         MXH_CODES_FENCE();
-        // c: slice (1, 0)
+        // c: slice (1, 0); the last reads of stage t
         read_a(stg, 1, 1, 1);
-        read_q(nstg + G::kA);
-        if constexpr (g == 3) read_head(t + 1);
         MXH_CODES_FENCE();
         multiply(1, 0, 0, FM::kPair);
         MXH_CODES_FENCE();
-        // d: slice (1, 1); the next step's first operands
+        // d: slice (1, 1); every wave has read the step's activations and the
+        // next step's are there: the slots are refilled and the next step's
+        // first operands read
+        wait_vm<G::ahead(g)>();
+        lds_barrier();
+        if constexpr (G::kWFirst && g % FM::kGR == 0) issue_w(t + FM::kGR, (g + FM::kGR) % 4 == 0);
+        issue_a(t + NST, slot);
+        if constexpr (!G::kWFirst && g % FM::kGR == 0) issue_w(t + FM::kGR, (g + FM::kGR) % 4 == 0);
+        read_q(t + 1, GN{});
+        if constexpr (g == 3) read_head(t + 1);
         read_a(nstg, 0, 0, 0);
         MXH_CODES_FENCE();
         multiply(1, 1, 1, false);
@@ -632,12 +678,13 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
         slot = nslot;
     };
 
+    issue_w(0, true);
 #pragma unroll
-    for (int st = 0; st < NST - 1; ++st) issue(st, st, st % 4 == 0);
-    wait_vm<G::ahead(0) + G::loads(NST - 2)>();
+    for (int st = 0; st < NST; ++st) issue_a(st, st);
+    wait_vm<(NST - 1) * G::kAL>();
     lds_barrier();
     read_head(0);
-    read_q(smem + G::kA);
+    read_q(0, C0{});
     read_a(smem, 0, 0, 0);
     block_d(0);
     decode(C0{}, C0{});
@@ -691,10 +738,12 @@ static int codes_launch(const CodesArgs& a, hipStream_t st) {
 template <int F>
 static int codes_tile(GemmTile t, const CodesArgs& a, hipStream_t st) {
     switch (t) {
-    case GT_128x256: return codes_launch<F, 2, 2, 2, 3>(a, st);
-    case GT_128x128: return codes_launch<F, 2, 2, 1, 3>(a, st);
-    case GT_64x256: return codes_launch<F, 1, 2, 1, 4>(a, st);
-    default: return codes_launch<F, 1, 1, 1, 5>(a, st);
+    case GT_128x256:
+        if constexpr (!Fmt<F>::kSplitW) return codes_launch<F, 2, 2, 2, 2>(a, st);
+        else return MXH_ERR_UNSUPPORTED;  // (two code operands: out of registers)
+    case GT_128x128: return codes_launch<F, 2, 2, 1, Fmt<F>::kGR == 2 ? 2 : 3>(a, st);
+    case GT_64x256: return codes_launch<F, 1, 2, 1, Fmt<F>::kGR == 2 ? 2 : 4>(a, st);
+    default: return codes_launch<F, 1, 1, 1, Fmt<F>::kGR == 2 ? 2 : 4>(a, st);
     }
 }
 
@@ -849,23 +898,26 @@ struct Plan {
 };
 
 // The tile shape and split of K with the lowest estimate of
-//   rounds of the 256 CUs x (steps of a work item x time of a step + start)
+//   rounds of the 256 CUs x (steps of a work item x time of a step + 7.5 us)
 //   + the reduction of the partial tiles,
 // the step's time lying between what it takes on a nearly idle chip and on a
-// full one (ns, measured per format and tile at K = 4096 .. 14336).
+// full one (ns, measured per format and tile at K = 4096 .. 14336, where the
+// estimate is within 10% of the measured time of the shapes tried); 7.5 us is
+// what a work item takes to start, fill its stages and store its outputs.
 Plan gemm_plan(int fmt, int m, int n, int k) {
     struct Cost {
         float idle, full;
     };
-    static const Cost cost[3][GT_COUNT] = {
-        {{1450.f, 2200.f}, {950.f, 1400.f}, {860.f, 1200.f}, {590.f, 900.f}},     // Q4_K, Q5_K
-        {{1900.f, 2450.f}, {1050.f, 1400.f}, {950.f, 1400.f}, {650.f, 1050.f}},   // Q8_0
-        {{2250.f, 3000.f}, {1400.f, 1750.f}, {1700.f, 2050.f}, {1600.f, 1750.f}}};  // Q6_K
+    static const Cost cost[4][GT_COUNT] = {
+        {{1420.f, 2130.f}, {830.f, 1160.f}, {800.f, 1110.f}, {490.f, 650.f}},       // Q4_K
+        {{1680.f, 2280.f}, {980.f, 1270.f}, {950.f, 1220.f}, {650.f, 830.f}},       // Q5_K
+        {{1720.f, 2300.f}, {980.f, 1180.f}, {950.f, 1200.f}, {600.f, 830.f}},       // Q8_0
+        {{1e6f, 1e6f}, {1430.f, 1730.f}, {1560.f, 1830.f}, {1000.f, 1130.f}}};      // Q6_K
     static const int bm[GT_COUNT] = {128, 128, 64, 32}, bn[GT_COUNT] = {256, 128, 256, 256};
-    const int cls = fmt == GF_Q80T ? 1 : fmt == GF_Q6KT ? 2 : 0, nblk = k / 256;
+    const int cls = fmt == GF_Q80T ? 2 : fmt == GF_Q6KT ? 3 : fmt == GF_Q5K || fmt == GF_Q5KT ? 1 : 0, nblk = k / 256;
     Plan best{GT_128x256, nblk, 1};
     double best_cost = 1e30;
-    for (int t = 0; t < GT_COUNT; ++t) {
+    for (int t = cls == 3 ? GT_128x128 : GT_128x256; t < GT_COUNT; ++t) {
         const int64_t tiles = (int64_t)((n + bn[t] - 1) / bn[t]) * ((m + bm[t] - 1) / bm[t]);
         for (int s = 1; s <= nblk && s <= 32; ++s) {
             const int blocks = (nblk + s - 1) / s;
@@ -875,7 +927,7 @@ Plan gemm_plan(int fmt, int m, int n, int k) {
             const int64_t items = tiles * s, rounds = (items + 255) / 256;
             const double load = items >= 256 ? 1.0 : items / 256.0;
             const Cost& c = cost[cls][t];
-            const double ns = rounds * (4.0 * blocks * (c.idle + load * (c.full - c.idle)) + 4000.0) +
+            const double ns = rounds * (4.0 * blocks * (c.idle + load * (c.full - c.idle)) + 7500.0) +
                               (s > 1 ? 3000.0 + floats * 4 / 3000.0 : 0.0);
             if (ns < best_cost) {
                 best_cost = ns;
