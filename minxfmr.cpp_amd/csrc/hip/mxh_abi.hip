@@ -142,6 +142,23 @@ int check_weight_ptr(int type, const void* w) {
     return MXH_OK;
 }
 
+// arguments of mxh_gemv, and its launch status as a status with a message
+int gemv_check(int type, const void* w, const float* x, const float* y, int64_t n, int64_t k) {
+    if (int rc = check_weight_ptr(type, w)) return rc;
+    if (!x || !y || !aligned(x, 16)) return set_error(MXH_ERR_ARG, "x must be non-null and 16-byte aligned");
+    if (type >= kTiledFlag && (type != (kTiledFlag | storage_type(type)) || tiled_type(storage_type(type), k) != type))
+        return set_error(MXH_ERR_ARG, "gemv: type %d is not the tiled form of rows of %lld columns", type, (long long)k);
+    if (n <= 0 || k <= 0 || row_bytes(type, k) == 0)
+        return set_error(MXH_ERR_ARG, "gemv: k=%lld is not a whole number of type-%d blocks", (long long)k, type);
+    return MXH_OK;
+}
+int gemv_status(int rc, int type, int64_t n, int64_t k) {
+    if (rc == MXH_ERR_ARG) return set_error(rc, "gemv: unsupported shape n=%lld k=%lld", (long long)n, (long long)k);
+    if (rc == MXH_ERR_UNSUPPORTED) return set_error(rc, "gemv: unsupported type %d", type);
+    if (rc) return set_error(rc, "gemv: launch failed");
+    return check_hip(hipGetLastError(), "gemv launch");
+}
+
 }  // namespace
 
 int set_error(int code, const char* fmt, ...) {
@@ -259,16 +276,8 @@ int mxh_timer_end(float* ms) {
 
 int mxh_gemv(int type, const void* w, const float* x, float* y, int64_t n, int64_t k, int form) {
     if (int rc = ensure_ready()) return rc;
-    if (int rc = check_weight_ptr(type, w)) return rc;
-    if (!x || !y || !aligned(x, 16)) return set_error(MXH_ERR_ARG, "x must be non-null and 16-byte aligned");
-    if (type >= kTiledFlag && (type != (kTiledFlag | storage_type(type)) || tiled_type(storage_type(type), k) != type))
-        return set_error(MXH_ERR_ARG, "gemv: type %d is not the tiled form of rows of %lld columns", type, (long long)k);
-    if (n <= 0 || k <= 0 || row_bytes(type, k) == 0)
-        return set_error(MXH_ERR_ARG, "gemv: k=%lld is not a whole number of type-%d blocks", (long long)k, type);
-    int rc = gemv_launch(type, w, x, y, nullptr, n, k, form, g_ctx.stream);
-    if (rc == MXH_ERR_ARG) return set_error(rc, "gemv: unsupported shape n=%lld k=%lld", (long long)n, (long long)k);
-    if (rc == MXH_ERR_UNSUPPORTED) return set_error(rc, "gemv: unsupported type %d", type);
-    return check_hip(hipGetLastError(), "gemv launch");
+    if (int rc = gemv_check(type, w, x, y, n, k)) return rc;
+    return gemv_status(gemv_launch(type, w, x, y, nullptr, n, k, form, g_ctx.stream), type, n, k);
 }
 
 static_assert(MXH_TILED_FLAG == kTiledFlag, "public and internal tiled flags differ");
@@ -289,8 +298,16 @@ int mxh_tile_rows(int type, void* w, int64_t rows, int64_t cols, int* tiled) {
 
 int mxh_matmul_rhs_t(int type, const float* a, int64_t m, const void* w, int64_t n, int64_t k, float* out, int form) {
     if (m <= 0) return set_error(MXH_ERR_ARG, "matmul: m must be positive");
-    for (int64_t i = 0; i < m; ++i)
-        if (int rc = mxh_gemv(type, w, a + i * k, out + i * n, n, k, form)) return rc;
+    if (m == 1) return mxh_gemv(type, w, a, out, n, k, form);
+    if (int rc = ensure_ready()) return rc;
+    if (int rc = gemv_check(type, w, a, out, n, k)) return rc;
+    if (n > INT32_MAX || k > INT32_MAX) return gemv_status(MXH_ERR_ARG, type, n, k);
+    constexpr int64_t kPart = 1 << 20;
+    for (int64_t i = 0; i < m; i += kPart)
+        if (int rc = gemv_status(gemv_rows_run(type, w, a + i * k, out + i * n, (int)(m - i < kPart ? m - i : kPart),
+                                               (int)n, (int)k, form, g_ctx.stream),
+                                 type, n, k))
+            return rc;
     return MXH_OK;
 }
 

@@ -1267,6 +1267,130 @@ __global__ __launch_bounds__(64 * W) void gemv_kernel(const uint8_t* pw, const f
     }
 }
 
+// ---- several rows of x at once -------------------------------------------
+//
+// y[i][n] = W[n] . x[i] for MB rows of x (mxh_matmul_rhs_t with m > 1).  The
+// weights are read and decoded once for all MB rows; every row of x is staged
+// as the GEMV stages it and meets the codes in the same arithmetic and order,
+// so the results are the GEMV's bit for bit.  Bound: at MB = 8 the v_dot4 work
+// of the rows (4096 x 4096 Q4_K: 3.4 us of VALU for 1.8 us of HBM) and the
+// staging (3 us of VALU per CU, every workgroup quantizes all MB rows), so
+// W = 8 waves share one staging per CU.  Measured against a loop of GEMVs
+// (us): see rows_launch.
+//
+// Thread t stages units (row b, elements 4 t + 256 W p, p < nb): kUnits loads at
+// a time are in flight before any is quantized.
+template <int W, int MB, bool INTX>
+__device__ __forceinline__ void stage_rows(float* smem, const float* __restrict__ x, int k, int rows, int stride) {
+    constexpr int kStep = 256 * W, kUnits = 16;
+    const int nb = (k + kStep - 1) / kStep, base = threadIdx.x * 4;
+    for (int b0 = 0, p0 = 0; b0 < MB;) {
+        float4 v[kUnits];
+        int b = b0, p = p0;  // (uniform)
+#pragma unroll
+        for (int i = 0; i < kUnits; ++i) {
+            const int e = base + p * kStep;
+            // rows past the last repeat it (never stored), elements past k are zero
+            v[i] = *reinterpret_cast<const float4*>(x + (size_t)min(b, rows - 1) * k + (e < k ? e : 0));
+            if (++p == nb) p = 0, ++b;
+        }
+        b = b0, p = p0;
+#pragma unroll
+        for (int i = 0; i < kUnits; ++i) {
+            if (b < MB) {
+                const int e = base + p * kStep;
+                float* dst = smem + (size_t)b * stride;
+                if constexpr (INTX) {
+                    const float4 u1[1] = {e < k ? v[i] : make_float4(0.f, 0.f, 0.f, 0.f)};
+                    quantize_units<W, 1>(u1, e, k, reinterpret_cast<uint32_t*>(dst));
+                } else if (e < k) {
+                    *reinterpret_cast<float4*>(dst + xpad(e)) = v[i];
+                }
+            }
+            if (++p == nb) p = 0, ++b;
+        }
+        b0 = b, p0 = p;
+    }
+    __syncthreads();
+}
+
+// dwords of LDS one staged row of x takes
+template <class Ty, int W>
+__host__ __device__ constexpr int rows_stride(int k) {
+    return Ty::kIntX ? xq_dwords<W>(k) : k + k / 16;
+}
+
+template <template <int> class T, int R, int MB, int W>
+__global__ __launch_bounds__(64 * W) void gemv_rows_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                           float* __restrict__ y, int n, int k, int rows, int form) {
+    using Ty = T<R>;
+    extern __shared__ float xs[];
+    const int stride = rows_stride<Ty, W>(k);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nchunks = k >> Ty::kChunkShift, cpl = (nchunks + 63) >> 6;
+    const size_t rb = row_bytes(Ty::kType, k);
+    const int n_groups = (n + R - 1) / R, n_waves = gridDim.x * W;
+    const auto view = [&](int b) {
+        if constexpr (Ty::kIntX) return xq_view<W>(xs + (size_t)b * stride, k);
+        else return (const float*)(xs + (size_t)b * stride);
+    };
+    typename Ty::Buf buf[2];
+    // step s of this wave: row group wave_id + (s / cpl) n_waves, chunk lane + 64 (s % cpl)
+    const int wave_id = blockIdx.x * W + wave;
+    const int my_groups = wave_id < n_groups ? (n_groups - 1 - wave_id) / n_waves + 1 : 0, total = my_groups * cpl;
+    // a step past the wave's last re-reads a few bytes of it: every step issues
+    // the same loads, so the waits count them exactly
+    int gi = 0, ji = 0;  // of the step issued
+    auto issue = [&](typename Ty::Buf& b) __attribute__((always_inline)) {
+        const bool past = gi >= my_groups;
+        const int grp = wave_id + (past ? my_groups - 1 : gi) * n_waves;
+        int rr[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) rr[r] = min(max(grp * R + r, 0), n - 1);
+        Ty::load(w, rb, rr, past ? 0 : min(lane + 64 * ji, nchunks - 1), b);
+        if (++ji == cpl) ji = 0, ++gi;
+    };
+    // the first step's weights are requested before the staging
+    issue(buf[0]);
+    stage_rows<W, MB, Ty::kIntX>(xs, x, k, rows, stride);
+    float acc[MB][R];
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[b][r] = 0.f;
+    int g = 0, j = 0;  // of the step consumed
+    auto consume = [&](const typename Ty::Buf& b) __attribute__((always_inline)) {
+        const int c = lane + 64 * j;
+        if (c < nchunks) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i) Ty::compute(b, c, view(i), form, acc[i]);
+        }
+        if (++j == cpl) {
+            const int n0 = (wave_id + g * n_waves) * R;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float v = wave_sum_lane63(acc[i][r]);
+                    if (lane == 63 && i < rows && n0 + r < n) y[(size_t)i * n + n0 + r] = v;
+                    acc[i][r] = 0.f;
+                }
+            }
+            j = 0;
+            ++g;
+        }
+    };
+    constexpr int kL = Ty::kLoads * R;
+    for (int s = 0; s < total; s += 2) {
+        issue(buf[1]);  // the step after the one consumed is in flight meanwhile
+        wait_vmcnt<kL>();
+        consume(buf[0]);
+        issue(buf[0]);
+        wait_vmcnt<kL>();
+        if (s + 1 < total) consume(buf[1]);
+    }
+}
+
 // Greedy id from the per-workgroup winners (minxfmr.cpp:2091-2115: the
 // largest logit, lowest index on ties); it becomes tokens[*pos + 1] and the
 // position advances.
@@ -1487,6 +1611,58 @@ bool launch_exact(const GemvArgs& a, int mode, hipStream_t st) {
     return steps == 1 && go(gemv_kernel<T, R, GEMV_PLAIN, 1, W>);
 }
 
+// Rows of x per launch of gemv_rows_kernel: what fits the LDS of a CU, at most 8
+// (a wave keeps 8 R sums).  W = 8 waves, one workgroup per CU: the staging is
+// paid once per CU.
+constexpr int kRowsWaves = 8;
+constexpr size_t kRowsLds = 160 * 1024;
+
+template <template <int> class T, int R, int MB>
+int rows_launch_mb(const uint8_t* w, const float* x, float* y, int n, int k, int rows, int form, hipStream_t st) {
+    auto kern = gemv_rows_kernel<T, R, MB, kRowsWaves>;
+    static bool attr_set = false;  // above 64 KiB of LDS needs the opt-in, once per kernel
+    if (!attr_set) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRowsLds) != hipSuccess)
+            return MXH_ERR_HIP;
+        attr_set = true;
+    }
+    const size_t lds = (size_t)MB * rows_stride<T<R>, kRowsWaves>(k) * 4;
+    const int groups = (n + R - 1) / R, wgs = (groups + kRowsWaves - 1) / kRowsWaves, n_cu = device_cus();
+    hipLaunchKernelGGL(kern, dim3((unsigned)(wgs < n_cu ? wgs : n_cu)), dim3(64 * kRowsWaves),
+                       lds, st, w, x, y, n, k, rows, form);
+    return MXH_OK;
+}
+
+// As many rows a launch as there are left and as 160 KiB of LDS holds (8 up to
+// 7000 inputs of a quantized type, 4 up to 14336), the next power of two where
+// fewer are left (its spare rows repeat the last and are not stored); a single
+// row left over is a GEMV.  One call against a loop of GEMVs, us:
+//   m x n x k       Q4_K         Q8_0 tiled   F16          F32
+//   2x1024x4096     6.5 / 10.4   6.4 / 9.0    11.6 / 14.2  27.6 / 31.8
+//   4x4096x4096     10.6 / 20.7  9.5 / 20.9   13.9 / 47.3  35.1 / 138
+//   8x4096x4096     16.4 / 41.1  14.9 / 41.4  18.3 / 92.6  38.3 / 275
+//   64x4096x4096    127 / 318    112 / 295    136 / 680    296 / 2143
+//   3x513x14336     29.7 / 44.6  25.3 / 37.3  47.3 / 49.9  116 / 116
+template <template <int> class T, int R, int MBMAX = 8>
+int rows_launch(const uint8_t* w, const float* x, float* y, int m, int n, int k, int form, hipStream_t st) {
+    const size_t row = (size_t)rows_stride<T<R>, kRowsWaves>(k) * 4;
+    const int fit = (int)(kRowsLds / row);
+    for (int i = 0; i < m;) {
+        const int left = m - i;
+        const float* xi = x + (size_t)i * k;
+        float* yi = y + (size_t)i * n;
+        int rc, used;
+        if (MBMAX >= 8 && left >= 5 && fit >= 8)
+            rc = rows_launch_mb<T, R, MBMAX>(w, xi, yi, n, k, used = left < 8 ? left : 8, form, st);
+        else if (left >= 3 && fit >= 4) rc = rows_launch_mb<T, R, 4>(w, xi, yi, n, k, used = left < 4 ? left : 4, form, st);
+        else if (left >= 2 && fit >= 2) rc = rows_launch_mb<T, R, 2>(w, xi, yi, n, k, used = 2, form, st);
+        else rc = gemv_launch(T<R>::kType, w, xi, yi, nullptr, n, k, form, st), used = 1;
+        if (rc) return rc;
+        i += used;
+    }
+    return MXH_OK;
+}
+
 }  // namespace
 
 // max K whose padded x fits the 64 KiB of LDS one workgroup may use
@@ -1541,6 +1717,28 @@ int gemv_run(int type, const GemvArgs& a, int mode, hipStream_t st) {
     case MXH_Q5_0: return launch_gemv<Q50, 4>(a, mode, st);
     case MXH_F16: return launch_gemv<F16W, 2>(a, mode, st);
     case MXH_F32: return launch_gemv<F32W, 2>(a, mode, st);
+    }
+    return MXH_ERR_UNSUPPORTED;
+}
+
+int gemv_rows_run(int type, const void* w, const float* x, float* y, int m, int n, int k, int form, hipStream_t st) {
+    if (k % 32 || k > kGemvMaxK || n <= 0 || m <= 0) return MXH_ERR_ARG;
+    const uint8_t* wb = (const uint8_t*)w;
+    switch (type) {
+    case MXH_Q4_K: return rows_launch<Q4K, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q4_K_TILED: return rows_launch<Q4KT, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q5_K: return rows_launch<Q5K, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q5_K_TILED: return rows_launch<Q5KT, 2>(wb, x, y, m, n, k, form, st);
+    // four rows at most: the nineteen loads of a raw Q6_K chunk in two buffers
+    // leave no registers for eight (spills: 107 us against 64 for eight GEMVs
+    // at 8x4096x4096; four rows 18.4 against 31.3)
+    case MXH_Q6_K: return rows_launch<Q6K, 1, 4>(wb, x, y, m, n, k, form, st);
+    case MXH_Q6_K_TILED: return rows_launch<Q6KT, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q8_0: return rows_launch<Q80, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q8_0_TILED: return rows_launch<Q80T, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_Q5_0: return rows_launch<Q50, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_F16: return rows_launch<F16W, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_F32: return rows_launch<F32W, 2>(wb, x, y, m, n, k, form, st);
     }
     return MXH_ERR_UNSUPPORTED;
 }

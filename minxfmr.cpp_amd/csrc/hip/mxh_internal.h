@@ -19,6 +19,10 @@ hipStream_t lib_stream();
 int gemv_launch(int type, const void* w, const float* x, float* y, const float* res, int64_t n, int64_t k, int form,
                 hipStream_t st);
 
+// y[m x n] = x[m x k] . W[n x k]^T for a few rows of x: several rows per pass
+// over the weights, in the GEMV's arithmetic (mxh_gemv.hip)
+int gemv_rows_run(int type, const void* w, const float* x, float* y, int m, int n, int k, int form, hipStream_t st);
+
 // Fused GEMV launch (see mxh_gemv.hip for the epilogues).
 enum { GEMV_PLAIN = 0, GEMV_SILU = 1, GEMV_ARGMAX = 2, GEMV_ATTN = 3 };
 struct GemvArgs {
