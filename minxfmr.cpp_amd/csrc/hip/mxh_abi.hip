@@ -6,6 +6,7 @@
 // the kernel's indexing assumes.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -29,7 +30,11 @@ struct Context {
     // grow-only staging buffers for host-pointer ops
     void* stage[4] = {nullptr, nullptr, nullptr, nullptr};
     size_t stage_bytes[4] = {0, 0, 0, 0};
+    // sampled ids, in pinned host memory; a call takes the next slot
+    int* sample_ids = nullptr;
+    std::atomic<unsigned> sample_calls{0};
 };
+constexpr unsigned kSampleSlots = 64;
 
 Context g_ctx;
 thread_local std::string g_err;
@@ -206,6 +211,8 @@ int mxh_init(int device) {
     if (int rc = check_hip(hipStreamCreateWithFlags(&g_ctx.stream, hipStreamNonBlocking), "hipStreamCreate")) return rc;
     if (int rc = check_hip(hipEventCreate(&g_ctx.ev0), "hipEventCreate")) return rc;
     if (int rc = check_hip(hipEventCreate(&g_ctx.ev1), "hipEventCreate")) return rc;
+    if (int rc = check_hip(hipHostMalloc((void**)&g_ctx.sample_ids, kSampleSlots * sizeof(int), hipHostMallocDefault), "hipHostMalloc"))
+        return rc;
     g_ctx.device = device;
     g_ctx.ready = true;
     return MXH_OK;
@@ -378,9 +385,8 @@ int mxh_sample(const float* logits, int n, int top_k, double temperature, double
     if (!logits || !token || n <= 0) return set_error(MXH_ERR_ARG, "sample: bad arguments");
     if (top_k < 1 || top_k > kSampleTopKMax || top_k > n)
         return set_error(MXH_ERR_ARG, "sample: top_k %d outside 1..min(%d, n)", top_k, kSampleTopKMax);
-    void *prm = nullptr, *cand = nullptr;
-    if (int rc = stage(0, sizeof(SampleParams) + sizeof(int), &prm)) return rc;
-    if (int rc = stage(1, sample_scratch_keys(n, top_k) * sizeof(uint64_t), &cand)) return rc;
+    void* cand = nullptr;
+    if (int rc = stage(1, sample_scratch_keys(n) * sizeof(uint64_t), &cand)) return rc;
     SampleParams h{};
     h.top_k = top_k;
     h.temperature = temperature;
@@ -388,15 +394,15 @@ int mxh_sample(const float* logits, int n, int top_k, double temperature, double
     h.min_p = min_p;
     h.seed = seed;
     h.draws = draw;
-    int* out = reinterpret_cast<int*>(static_cast<char*>(prm) + sizeof(SampleParams));
-    if (int rc = check_hip(hipMemcpyAsync(prm, &h, sizeof(h), hipMemcpyHostToDevice, g_ctx.stream), "sample params"))
-        return rc;
-    if (int rc = sample_launch(logits, n, static_cast<SampleParams*>(prm), top_k, static_cast<uint64_t*>(cand), out,
-                               nullptr, nullptr, g_ctx.stream))
+    int* id = g_ctx.sample_ids + g_ctx.sample_calls.fetch_add(1, std::memory_order_relaxed) % kSampleSlots;
+    // parameters by value and the id straight to pinned host memory: no copies
+    if (int rc = sample_launch(logits, n, nullptr, &h, top_k, static_cast<uint64_t*>(cand), id, nullptr, nullptr,
+                               g_ctx.stream))
         return set_error(rc, "sample: vocabulary of %d too large for top_k %d", n, top_k);
-    if (int rc = check_hip(hipMemcpyAsync(token, out, sizeof(int), hipMemcpyDeviceToHost, g_ctx.stream), "sample id"))
-        return rc;
-    return check_hip(hipStreamSynchronize(g_ctx.stream), "sample");
+    if (int rc = check_hip(hipGetLastError(), "sample launch")) return rc;
+    if (int rc = check_hip(hipStreamSynchronize(g_ctx.stream), "sample")) return rc;
+    *token = *id;
+    return MXH_OK;
 }
 
 int mxh_preload(const void* host, size_t bytes) {

@@ -147,9 +147,8 @@ struct SampleParams {
     uint64_t seed;
     uint64_t draws;
 };
-size_t sample_scratch_keys(int n, int top_k);
-// largest top_k the device sampler takes (two passes up to 64, a one-
-// workgroup radix select above)
+size_t sample_scratch_keys(int n);
+// largest top_k the device sampler takes
 constexpr int kSampleTopKMax = 4096;
 // Logit edits before the choice (minxfmr.cpp:2047-2089), parameters in
 // device memory: suppressed ids to -inf, then over the last last_n ids of
@@ -163,8 +162,9 @@ struct EditParams {
 };
 int logit_edits_launch(float* logits, int n_vocab, const int* tokens, const int* pos, const EditParams* prm,
                        const int* suppress, int* cnt, hipStream_t st);
-int sample_launch(const float* logits, int n, SampleParams* prm, int top_k, uint64_t* cand, int* out, int* tokens,
-                  int* pos, hipStream_t st);
+// with prm its parameters (device memory), else *call's
+int sample_launch(const float* logits, int n, SampleParams* prm, const SampleParams* call, int top_k, uint64_t* cand,
+                  int* out, int* tokens, int* pos, hipStream_t st);
 int qkv_prep_rows_launch(const float* qkv, int ldq, const float* bias, const float* q_norm, const float* k_norm,
                          const double* rope_cs, int p0, int m, float* q_out, __half* kc, __half* vc, int nh, int nkv,
                          int hd, int neox, float eps, hipStream_t st);

@@ -214,7 +214,7 @@ int enqueue_step(mxh_model* m, bool with_head, bool wrapped, hipStream_t st) {
             if (m->edits)
                 rc |= logit_edits_launch(m->logits, c.n_vocab, m->tokens, m->pos, m->eprm, m->esup, m->ecnt, st);
             if (m->sampling) {
-                rc |= sample_launch(m->logits, c.n_vocab, m->sprm, m->top_k, m->scand, nullptr, m->tokens, m->pos, st);
+                rc |= sample_launch(m->logits, c.n_vocab, m->sprm, nullptr, m->top_k, m->scand, nullptr, m->tokens, m->pos, st);
             } else {
                 rc |= argmax_launch(m->logits, c.n_vocab, m->tokens, m->pos, st);
                 rc |= add_int_launch(m->pos, 1, st);
@@ -649,7 +649,7 @@ static int model_open_impl(const char* gguf_path, int n_ctx, int flags, mxh_mode
     if (!rc) rc = dalloc(&m->red_val, (size_t)m->red_cap);
     if (!rc) rc = dalloc(&m->red_idx, (size_t)m->red_cap);
     if (!rc) rc = dalloc(&m->sprm, 1);
-    if (!rc) rc = dalloc(&m->scand, std::max(sample_scratch_keys(c.n_vocab, 64), (size_t)4096));
+    if (!rc) rc = dalloc(&m->scand, sample_scratch_keys(c.n_vocab));
     if (!rc) rc = check_hip(hipMemset(m->sprm, 0, sizeof(SampleParams)), "sampler init");
     if (!rc) rc = dalloc(&m->eprm, 1);
     if (!rc) rc = dalloc(&m->esup, (size_t)c.n_vocab);

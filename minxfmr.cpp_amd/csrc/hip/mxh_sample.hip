@@ -1,19 +1,26 @@
 // mxh_sample.hip — top-k / temperature / top-p / min-p sampling on the device
 // (reference: src/api/minxfmr.cpp:2091-2171, with a seeded draw).
 //
-// top_k up to 64, two passes.  Pass 1: each of W workgroups sorts its slice of the logits in LDS (bitonic,
-// 64-bit keys: order-preserving bits of the logit above the complemented id,
-// so ties go to the lower id, as the reference's partial_sort with `>` and an
-// increasing initial order) and keeps its best kk = pow2(top_k) candidates.
-// Pass 2: one workgroup sorts the lists of the top_k groups with the largest
-// maxima (they hold every candidate that can rank in the top k), then thread
-// 0 forms the probabilities in double exactly as the reference does (exp of
+// Keys: order-preserving bits of the logit above the complemented id, so ties
+// go to the lower id, as the reference's partial_sort with `>` and an
+// increasing initial order.  Pass 1, the whole chip: the largest logit of
+// every group of 4 to 16 neighbouring ids (more above 196,608 ids).  Pass 2,
+// one workgroup: the k-th largest group maximum T bounds the k-th largest key
+// from below (k maxima reach it) and only groups whose maximum reaches it hold
+// keys at or above it, so the logits of about k groups are read again, the
+// hardly more than k keys at or above T are sorted, and the choice is made
+// among the first k in double exactly as the reference makes it (exp of
 // (l - max) / T, normalise, top-p cut and renormalise, min-p cut and
-// renormalise) and draws.  top_k from 65 to 4096: one workgroup selects the
-// k best keys by a radix select, sorts them and chooses the same way.  The
-// uniform of draw d is splitmix64 at state
-// seed + (d + 1) * 0x9E3779B97F4A7C15, the d-th value of the sequence that
-// starts at `seed`.
+// renormalise).  Where more than kCandMax keys reach T (many equal logits, or
+// large logits side by side), T is raised over the keys themselves first.
+//
+// Bound: the one workgroup's chain of barriers and LDS latencies, two launches
+// and the wait for the id.  Selecting by sorting (64 lists sorted in LDS, then
+// 4,096 keys by one workgroup) took 156 us for top_k 40 of 151,936 ids with
+// the copies of its parameters and of the id; this 34.
+//
+// The uniform of draw d is splitmix64 at state seed + (d + 1) *
+// 0x9E3779B97F4A7C15, the d-th value of the sequence that starts at `seed`.
 #include <hip/hip_runtime.h>
 
 #include "mxh_device.h"
@@ -23,57 +30,53 @@ namespace mxh {
 
 namespace {
 
-constexpr int kSortMax = 4096;  // keys one workgroup sorts in LDS
-constexpr int kTopKMax = 64;      // the two-pass form
-constexpr int kTopKLarge = kSampleTopKMax;  // the one-workgroup radix-select form
-constexpr int kMaxGroups = 2048;  // pass-1 lists one pass-2 workgroup ranks
+constexpr int kCandMax = kSampleTopKMax;  // keys the workgroup sorts
+constexpr int kThreads = 1024, kWaves = kThreads / 64;
+constexpr int kGroupRegs = 12;  // group maxima a thread of pass 2 holds
+constexpr int kGroupsMax = kThreads * kGroupRegs;
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any float address
+
+__device__ __forceinline__ uint32_t order_bits(float v) {
+    const uint32_t u = __float_as_uint(v);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return 0u;  // NaN sorts last
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
 
 __device__ __forceinline__ uint64_t sort_key(float v, int idx) {
-    uint32_t u = __float_as_uint(v);
-    if ((u & 0x7fffffffu) > 0x7f800000u) u = 0u;  // NaN sorts last
-    else u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-    return ((uint64_t)u << 32) | (uint32_t)(~(uint32_t)idx);
+    return ((uint64_t)order_bits(v) << 32) | (uint32_t)(~(uint32_t)idx);
 }
 
 __device__ __forceinline__ int key_id(uint64_t k) { return (int)(~(uint32_t)(k & 0xffffffffu)); }
 
-// descending bitonic sort of s[0 .. p), p a power of two
-__device__ void bitonic_desc(uint64_t* s, int p) {
-    for (int k = 2; k <= p; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < p; i += blockDim.x) {
-                const int ixj = i ^ j;
-                if (ixj > i) {
-                    const uint64_t a = s[i], b = s[ixj];
-                    const bool desc = (i & k) == 0;
-                    if (desc ? (a < b) : (a > b)) {
-                        s[i] = b;
-                        s[ixj] = a;
-                    }
-                }
+// ids per group: the fewest (a power of two, four at least) that leave at most
+// kGroupsMax groups
+int group_shift(int n) {
+    int g = 2;
+    while ((((int64_t)n + (1ll << g) - 1) >> g) > kGroupsMax) ++g;
+    return g;
+}
+int group_count(int n) { return (int)(((int64_t)n + (1ll << group_shift(n)) - 1) >> group_shift(n)); }
+
+// 1, 2 or 4 lanes per group (1 << lsh), four ids a load
+__global__ __launch_bounds__(256) void group_max_kernel(const float* __restrict__ logits, int n, int gsh, int lsh,
+                                                        int groups, uint32_t* __restrict__ gmax) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, g = t >> lsh;
+    uint32_t m = 0u;
+    if (g < groups) {
+        const int64_t end = (g + 1) << gsh;
+        for (int64_t e = (g << gsh) + 4 * (t & ((1 << lsh) - 1)); e < end && e < n; e += 4 << lsh) {
+            if (e + 4 <= n) {
+                const f32x4u v = *reinterpret_cast<const f32x4u*>(logits + e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) m = max(m, order_bits(v[i]));
+            } else {
+                for (int64_t i = e; i < n; ++i) m = max(m, order_bits(logits[i]));
             }
-            __syncthreads();
         }
-}
-
-__device__ __forceinline__ int pow2_at_least(int v) {
-    int p = 1;
-    while (p < v) p <<= 1;
-    return p;
-}
-
-__global__ __launch_bounds__(1024) void topk_pass1_kernel(const float* __restrict__ logits, int n, int slice, int kk,
-                                                          uint64_t* __restrict__ cand) {
-    __shared__ uint64_t s[kSortMax];
-    const int b0 = blockIdx.x * slice, b1 = min(n, b0 + slice);
-    const int p = pow2_at_least(slice > kk ? slice : kk);  // short slices pad up to the list length
-    for (int i = threadIdx.x; i < p; i += blockDim.x) {
-        const int idx = b0 + i;
-        s[i] = idx < b1 ? sort_key(logits[idx], idx) : 0ull;
     }
-    __syncthreads();
-    bitonic_desc(s, p);
-    for (int i = threadIdx.x; i < kk; i += blockDim.x) cand[(size_t)blockIdx.x * kk + i] = s[i];
+    for (int off = 1; off < 1 << lsh; off <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+    if (g < groups && (t & ((1 << lsh) - 1)) == 0) gmax[g] = m;
 }
 
 __device__ __forceinline__ double draw_uniform(uint64_t seed, uint64_t d) {
@@ -84,208 +87,311 @@ __device__ __forceinline__ double draw_uniform(uint64_t seed, uint64_t d) {
     return (double)(z >> 11) * (1.0 / 9007199254740992.0);
 }
 
-// The choice among the k best ids in order (ids[0 .. k)), as the reference
-// makes it (minxfmr.cpp:2104-2171): the k unnormalised probabilities
-// exp((l - max) / T) in double, computed by the workgroup into pr, then in
-// thread 0, in the reference's order: normalise, top-p cut and renormalise,
-// min-p cut and renormalise, and the draw.  The token goes to out[0] or,
-// with tokens/pos, to tokens[*pos + 1] with the position advanced (the
-// decode loop on the device); the draw counter advances either way.
-// Called by every thread of the workgroup.
-__device__ void choose(const float* __restrict__ logits, const int* ids, int k, double* pr, SampleParams* prm,
-                       int* out, int* tokens, int* pos) {
-    const double temperature = prm->temperature;
-    if (temperature > 0.0) {
-        const double mx = logits[ids[0]];
-        for (int i = threadIdx.x; i < k; i += blockDim.x) pr[i] = exp(((double)logits[ids[i]] - mx) / temperature);
+// p[0] + p[1] + ... in that order: the loads of a stretch are issued together,
+// only the additions form a chain
+__device__ __forceinline__ double sum_in_order(const double* p, int m) {
+    double s = 0.0;
+#pragma unroll 16
+    for (int i = 0; i < m; ++i) s += p[i];
+    return s;
+}
+
+// First i with reached(p[0] + .. + p[i]) for non-negative p, m - 1 if none;
+// *cum is that sum.  Whole stretches first (the sums only grow), then the one
+// that holds it again.
+template <class F>
+__device__ __forceinline__ int first_reaching(const double* p, int m, F&& reached, double* cum) {
+    double c = 0.0;
+    int i = 0;
+    for (; i + 16 <= m; i += 16) {
+        double c1 = c;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) c1 += p[i + j];
+        if (reached(c1)) break;
+        c = c1;
     }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double top_p = prm->top_p, min_p = prm->min_p;
-    int pick = ids[0];
-    if (temperature > 0.0) {
+    for (; i < m; ++i) {
+        c += p[i];
+        if (reached(c)) break;
+    }
+    *cum = c;
+    return i < m ? i : m - 1;
+}
+
+// The choice among the k best ids in order (ids[0 .. k)), as the reference
+// makes it (minxfmr.cpp:2104-2171), in double: exponentials and divisions by
+// the whole workgroup, the sums by thread 0 in the reference's order.  The
+// token goes to out[0] or, with tokens/pos, to tokens[*pos + 1] with the
+// position advanced (the decode loop on the device); with prm the draw counter
+// advances.  Called by every thread of the workgroup.
+__device__ void choose(const float* __restrict__ logits, const int* ids, int k, double* pr, const SampleParams& sp,
+                       SampleParams* prm, int* out, int* tokens, int* pos) {
+    __shared__ double val;
+    __shared__ int cut;
+    const int tid = threadIdx.x;
+    int pick = 0, m = k;  // pick: index into ids
+    if (sp.temperature > 0.0) {
+        double top_p = sp.top_p, min_p = sp.min_p;
         if (top_p <= 0.0 || top_p > 1.0) top_p = 1.0;
         if (min_p < 0.0) min_p = 0.0;
         if (min_p > 1.0) min_p = 1.0;
-        double sum = 0.0;
-        for (int i = 0; i < k; ++i) sum += pr[i];
+        const double mx = logits[ids[0]];
+        for (int i = tid; i < k; i += kThreads) pr[i] = exp(((double)logits[ids[i]] - mx) / sp.temperature);
+        __syncthreads();
+        const auto divide = [&](double by) {  // pr[0 .. m) /= by
+            for (int i = tid; i < m; i += kThreads) pr[i] /= by;
+            __syncthreads();
+        };
+        if (tid == 0) val = sum_in_order(pr, m);
+        __syncthreads();
+        const double sum = val;
         if (sum > 0.0) {
-            for (int i = 0; i < k; ++i) pr[i] /= sum;
-            int m = k;
+            divide(sum);
             if (top_p < 1.0) {
-                double cum = 0.0;
-                m = 0;
-                for (int i = 0; i < k; ++i) {
-                    cum += pr[i];
-                    m = i + 1;
-                    if (cum >= top_p) break;
-                }
-                double r = 0.0;
-                for (int i = 0; i < m; ++i) r += pr[i];
-                if (r > 0.0)
-                    for (int i = 0; i < m; ++i) pr[i] /= r;
+                if (tid == 0) cut = first_reaching(pr, k, [&](double c) { return c >= top_p; }, &val) + 1;
+                __syncthreads();
+                m = cut;
+                const double r = val;  // the sum of the kept, in the same order
+                if (r > 0.0) divide(r);
             }
             if (min_p > 0.0 && m > 1) {
                 const double thr = pr[0] * min_p;
-                int keep = 1;
-                for (int i = 1; i < m; ++i) {
-                    if (pr[i] >= thr) keep = i + 1;
-                    else break;
-                }
-                m = keep;
-                double r = 0.0;
-                for (int i = 0; i < m; ++i) r += pr[i];
-                if (r > 0.0)
-                    for (int i = 0; i < m; ++i) pr[i] /= r;
+                if (tid == 0) cut = m;
+                __syncthreads();
+                for (int i = 1 + tid; i < m; i += kThreads)
+                    if (!(pr[i] >= thr)) {
+                        atomicMin(&cut, i);
+                        break;
+                    }
+                __syncthreads();
+                m = cut;
+                if (tid == 0) val = sum_in_order(pr, m);
+                __syncthreads();
+                const double r = val;
+                if (r > 0.0) divide(r);
             }
-            double total = 0.0;
-            for (int i = 0; i < m; ++i) total += pr[i];
-            const double u = draw_uniform(prm->seed, prm->draws) * total;
-            double cum = 0.0;
-            pick = ids[m - 1];
-            for (int i = 0; i < m; ++i) {
-                cum += pr[i];
-                if (u < cum) {
-                    pick = ids[i];
-                    break;
-                }
+            if (tid == 0) {
+                const double u = draw_uniform(sp.seed, sp.draws) * sum_in_order(pr, m);
+                double c;
+                pick = first_reaching(pr, m, [&](double v) { return u < v; }, &c);
             }
         }
-        prm->draws += 1;
     }
-    if (out) out[0] = pick;
+    if (tid != 0) return;
+    if (prm && sp.temperature > 0.0) prm->draws = sp.draws + 1;
+    if (out) out[0] = ids[pick];
     if (tokens) {
         const int q = *pos;
-        tokens[q + 1] = pick;
+        tokens[q + 1] = ids[pick];
         *pos = q + 1;
     }
 }
 
-// Pass 2 (top_k <= kTopKMax): candidates -> token.
-//
-// Each group's list is sorted, so its first key is the group's maximum.  The
-// k-th largest group maximum T bounds the k-th largest key from below (k
-// group maxima reach it), and only the k groups whose maximum reaches T can
-// hold keys >= T: their lists are the only ones sorted.  Keys are distinct
-// (they carry the id), so the order is the full sort's.
-__global__ __launch_bounds__(1024) void topk_pass2_kernel(const float* __restrict__ logits, const uint64_t* cand,
-                                                          int groups, int kk, SampleParams* prm, int* out,
-                                                          int* tokens, int* pos) {
-    __shared__ uint64_t s[kSortMax];
-    __shared__ uint64_t gmax[kMaxGroups];
-    __shared__ double pr[kTopKMax];
-    __shared__ int ids[kTopKMax];
-    const int k = prm->top_k;
-    for (int j = threadIdx.x; j < groups; j += blockDim.x) gmax[j] = cand[(size_t)j * kk];
-    __syncthreads();
-    const int sel = groups < k ? groups : k;  // groups taken
-    for (int j = threadIdx.x; j < groups; j += blockDim.x) {
-        const uint64_t v = gmax[j];
-        int rank = 0;
-        for (int i = 0; i < groups; ++i) rank += gmax[i] > v;
-        if (rank < sel)
-            for (int i = 0; i < kk; ++i) s[rank * kk + i] = cand[(size_t)j * kk + i];
-    }
-    const int p = pow2_at_least(sel * kk);
-    for (int i = sel * kk + threadIdx.x; i < p; i += blockDim.x) s[i] = 0ull;
-    __syncthreads();
-    bitonic_desc(s, p);
-    for (int i = threadIdx.x; i < k; i += blockDim.x) ids[i] = key_id(s[i]);
-    __syncthreads();
-    choose(logits, ids, k, pr, prm, out, tokens, pos);
+// descending over the wave's lanes
+__device__ __forceinline__ uint64_t sort64_desc(uint64_t v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            const uint64_t o = (uint64_t)__shfl_xor((unsigned long long)v, j, 64);
+            // the lower lane of a pair keeps the larger key in a descending run
+            const bool larger = ((lane & k) == 0) == ((lane & j) == 0);
+            v = (o > v) == larger ? o : v;
+        }
+    return v;
 }
 
-// top_k in (kTopKMax, kTopKLarge]: one workgroup finds the k-th largest key T
-// by a radix select over the 64-bit keys (8-bit digits, most significant
-// first: per digit a histogram of the keys that share the digits chosen so
-// far, then the digit whose bin holds the k-th), gathers the k keys >= T
-// (exactly k: keys are distinct), sorts them and chooses as pass 2 does.
-// Same keys, same order, same choice as the two-pass form.
-__global__ __launch_bounds__(1024) void topk_large_kernel(const float* __restrict__ logits, int n, SampleParams* prm,
-                                                          int* out, int* tokens, int* pos) {
-    __shared__ uint64_t s[kTopKLarge];  // the k keys, then their probabilities (doubles)
-    __shared__ int ids[kTopKLarge];
-    __shared__ unsigned hist[256];
-    __shared__ uint64_t prefix_s;
-    __shared__ int need_s, count_s;
-    const int k = prm->top_k;
-    uint64_t prefix = 0;
-    int need = k;
-    for (int shift = 56; shift >= 0; shift -= 8) {
-        for (int b = threadIdx.x; b < 256; b += blockDim.x) hist[b] = 0u;
+// keys of a descending run of 64 that are larger than v
+__device__ __forceinline__ int run_larger(const uint64_t* run, uint64_t v) {
+    int lo = 0;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1)
+        if (run[lo + step - 1] > v) lo += step;
+    return lo + (run[lo] > v);
+}
+
+// prm: parameters in device memory, or null for `call`'s
+__global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __restrict__ logits, int n, int gsh,
+                                                               int groups, const uint32_t* __restrict__ gmax,
+                                                               SampleParams* prm, SampleParams call, int* out,
+                                                               int* tokens, int* pos) {
+    __shared__ __attribute__((aligned(16))) uint64_t s[kCandMax];  // keys, then the probabilities (doubles)
+    __shared__ __attribute__((aligned(16))) uint16_t list[kGroupsMax];  // groups taken, then the ids in order
+    __shared__ int part[2][4][kWaves];
+    __shared__ int n_list, n_cand;
+    __shared__ uint32_t top;
+    static_assert(sizeof(list) >= kCandMax * sizeof(int) && kGroupsMax <= 65536, "");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const SampleParams sp = prm ? *prm : call;
+    const int k = sp.top_k;
+
+    uint32_t mx[kGroupRegs];
+    uint32_t my_top = 0u;
+#pragma unroll
+    for (int r = 0; r < kGroupRegs; ++r) {
+        const int g = tid + kThreads * r;
+        mx[r] = g < groups ? gmax[g] : 0u;
+        my_top = max(my_top, mx[r]);
+    }
+    if (tid == 0) n_list = 0, n_cand = 0, top = 0u;
+    // per-wave counts -> the workgroup's (part is double-buffered: one barrier a call)
+    int turn = 0;
+    const auto total3 = [&](int a, int b, int c, int (&t)[3]) {
+        if (lane == 0) part[turn][0][wave] = a, part[turn][1][wave] = b, part[turn][2][wave] = c;
         __syncthreads();
-        const uint64_t hi_mask = shift == 56 ? 0ull : ~0ull << (shift + 8);
-        for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            const uint64_t key = sort_key(logits[i], i);
-            if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1u);
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int above = 0, b = 255;
-            for (; b > 0; --b) {
-                if (above + (int)hist[b] >= need) break;
-                above += (int)hist[b];
+        t[0] = t[1] = t[2] = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+            t[0] += part[turn][0][w], t[1] += part[turn][1][w], t[2] += part[turn][2][w];
+        turn ^= 1;
+    };
+
+    // T: the k-th largest group maximum, from the top bit down, or a value
+    // below it that few more maxima reach; 0 (every key) with fewer groups
+    uint32_t T = 0u;
+    if (groups >= k)
+        for (int bit = 31; bit >= 0; --bit) {
+            const uint32_t c = T | (1u << bit);
+            int cnt = 0;
+#pragma unroll
+            for (int r = 0; r < kGroupRegs; ++r) cnt += __popcll(__ballot(mx[r] >= c));
+            if (lane == 0) part[turn][0][wave] = cnt;
+            __syncthreads();
+            int t = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) t += part[turn][0][w];
+            turn ^= 1;
+            if (t >= k) {
+                T = c;
+                if (t <= k + (k >> 3)) break;
             }
-            prefix_s = prefix | ((uint64_t)b << shift);
-            need_s = need - above;
-            count_s = 0;
+        }
+    __syncthreads();
+
+    // the groups whose maximum reaches T
+#pragma unroll
+    for (int r = 0; r < kGroupRegs; ++r) {
+        const int g = tid + kThreads * r;
+        const bool in = g < groups && mx[r] >= T;
+        const uint64_t mask = __ballot(in);
+        if (!mask) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&n_list, __popcll(mask));
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (in) list[base + __popcll(mask & ((1ull << lane) - 1))] = (uint16_t)g;
+    }
+    atomicMax(&top, my_top);
+    __syncthreads();
+
+    // f(key, valid) over their ids, whole waves at a time
+    const int64_t n_ids = (int64_t)n_list << gsh;
+    const auto each = [&](auto&& f) {
+        for (int64_t i = tid; i - lane < n_ids; i += kThreads) {
+            const int64_t e = i < n_ids ? ((int64_t)list[i >> gsh] << gsh) + (i & ((1 << gsh) - 1)) : n;
+            f(e < n ? sort_key(logits[e], (int)e) : 0ull);
+        }
+    };
+    // the keys >= t to s (as many as fit); every real key is larger than zero
+    const auto gather = [&](uint64_t t) {
+        each([&](uint64_t key) {
+            const bool in = key >= t && key != 0ull;
+            const uint64_t mask = __ballot(in);
+            if (!mask) return;
+            int base = 0;
+            if (lane == 0) base = atomicAdd(&n_cand, __popcll(mask));
+            const int at = __builtin_amdgcn_readfirstlane(base) + __popcll(mask & ((1ull << lane) - 1));
+            if (in && at < kCandMax) s[at] = key;
+        });
+        __syncthreads();
+    };
+    gather((uint64_t)T << 32);
+    if (n_cand > kCandMax) {
+        // The k-th largest key, or one below it that at most kCandMax reach:
+        // two bits a pass.  It lies between T and the largest maximum, so the
+        // value bits above their first difference are known; then the id's.
+        int id_bits = 1;
+        while (id_bits < 31 && (n >> id_bits)) ++id_bits;
+        const uint32_t diff = T ^ top;
+        const int vbits = diff ? 32 - __builtin_clz(diff) : 0;
+        uint64_t t = (uint64_t)(vbits < 32 ? T >> vbits << vbits : 0u) << 32;
+        int reach = n_cand;
+        const auto narrow = [&](int bits, int low) {
+            for (int hi = bits; hi > 0 && reach > kCandMax; hi -= 2) {
+                const int sh = low + (hi > 1 ? hi - 2 : 0), steps = hi > 1 ? 3 : 1;
+                const uint64_t c1 = t + (1ull << sh), c2 = t + (2ull << sh), c3 = t + (3ull << sh);
+                int a = 0, b = 0, c = 0;
+                each([&](uint64_t key) {
+                    a += __popcll(__ballot(key >= c1));
+                    b += __popcll(__ballot(key >= c2));
+                    c += __popcll(__ballot(key >= c3));
+                });
+                int cnt[3];
+                total3(a, b, c, cnt);
+                for (int j = 0; j < steps; ++j)
+                    if (cnt[j] >= k) t += 1ull << sh, reach = cnt[j];
+            }
+        };
+        narrow(vbits, 32);
+        if (reach > kCandMax) {
+            t |= 0xffffffffull & (~0ull << id_bits);  // an id's complement has these bits set
+            narrow(id_bits, 0);
         }
         __syncthreads();
-        prefix = prefix_s;
-        need = need_s;
+        if (tid == 0) n_cand = 0;
+        __syncthreads();
+        gather(t);
     }
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const uint64_t key = sort_key(logits[i], i);
-        if (key >= prefix) s[atomicAdd(&count_s, 1)] = key;
+
+    // Sorted runs of 64, one a wave; a key's place is its place in its own run
+    // plus the larger keys of every other run (keys are distinct).
+    const int cand = n_cand, runs = (cand + 63) >> 6;
+    int* ids = reinterpret_cast<int*>(list);
+    constexpr int kRunRegs = kCandMax / kThreads;
+    uint64_t key[kRunRegs];
+#pragma unroll
+    for (int r = 0; r < kRunRegs; ++r) {
+        const int i = tid + kThreads * r;
+        if (wave + kWaves * r < runs) {
+            key[r] = sort64_desc(i < cand ? s[i] : 0ull);
+            s[i] = key[r];
+        }
     }
-    const int p = pow2_at_least(k);
     __syncthreads();
-    for (int i = k + threadIdx.x; i < p; i += blockDim.x) s[i] = 0ull;
+#pragma unroll
+    for (int r = 0; r < kRunRegs; ++r) {
+        const int run = wave + kWaves * r;
+        if (run < runs) {
+            int at = lane;
+            for (int q = 0; q < runs; ++q)
+                if (q != run) at += run_larger(s + 64 * q, key[r]);
+            if (key[r] && at < k) ids[at] = key_id(key[r]);
+        }
+    }
     __syncthreads();
-    bitonic_desc(s, p);
-    for (int i = threadIdx.x; i < k; i += blockDim.x) ids[i] = key_id(s[i]);
-    __syncthreads();
-    choose(logits, ids, k, reinterpret_cast<double*>(s), prm, out, tokens, pos);
+    choose(logits, ids, k, reinterpret_cast<double*>(s), sp, prm, out, tokens, pos);
 }
 
 }  // namespace
 
-// Pass-1 workgroups and the per-workgroup list length for n logits and
-// top_k: the candidates of all workgroups must fit one LDS sort.
-void sample_shape(int n, int top_k, int* groups, int* slice, int* kk) {
-    int k2 = 1;
-    while (k2 < top_k) k2 <<= 1;
-    int w = kSortMax / k2;
-    if (w > 256) w = 256;
-    int sl = (n + w - 1) / w;
-    while (sl > kSortMax) {  // very large vocabularies: fewer, larger lists are not possible
-        w *= 2;
-        sl = (n + w - 1) / w;
-    }
-    *groups = (n + sl - 1) / sl;
-    *slice = sl;
-    *kk = k2;
-}
+size_t sample_scratch_keys(int n) { return ((size_t)group_count(n) + 1) / 2; }
 
-size_t sample_scratch_keys(int n, int top_k) {
-    if (top_k > kTopKMax) return 1;  // the radix-select form needs no candidate lists
-    int g, sl, kk;
-    sample_shape(n, top_k, &g, &sl, &kk);
-    return (size_t)g * kk;
-}
-
-int sample_launch(const float* logits, int n, SampleParams* prm, int top_k, uint64_t* cand, int* out, int* tokens,
-                  int* pos, hipStream_t st) {
-    if (n <= 0 || top_k < 1 || top_k > kTopKLarge || top_k > n) return MXH_ERR_ARG;
-    if (top_k > kTopKMax) {
-        hipLaunchKernelGGL(topk_large_kernel, dim3(1), dim3(1024), 0, st, logits, n, prm, out, tokens, pos);
-        return MXH_OK;
+// Vocabularies taken: any for top_k above 64, else up to 4096 times 4096 /
+// top_k (to the next power of two) ids, 8M at most.
+int sample_launch(const float* logits, int n, SampleParams* prm, const SampleParams* call, int top_k, uint64_t* cand,
+                  int* out, int* tokens, int* pos, hipStream_t st) {
+    if (n <= 0 || top_k < 1 || top_k > kSampleTopKMax || top_k > n) return MXH_ERR_ARG;
+    if (top_k <= 64) {
+        int64_t lists = 4096;
+        while (lists * top_k > 4096) lists >>= 1;
+        if (n > 4096 * (lists < 2048 ? lists : 2048)) return MXH_ERR_UNSUPPORTED;
     }
-    int g, sl, kk;
-    sample_shape(n, top_k, &g, &sl, &kk);
-    if ((size_t)g * kk > (size_t)kSortMax || g > kMaxGroups) return MXH_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(topk_pass1_kernel, dim3(g), dim3(1024), 0, st, logits, n, sl, kk, cand);
-    hipLaunchKernelGGL(topk_pass2_kernel, dim3(1), dim3(1024), 0, st, logits, cand, g, kk, prm, out, tokens, pos);
+    const int gsh = group_shift(n), lsh = gsh < 4 ? gsh - 2 : 2, groups = group_count(n);
+    uint32_t* gmax = reinterpret_cast<uint32_t*>(cand);
+    hipLaunchKernelGGL(group_max_kernel, dim3((unsigned)(((int64_t)(groups << lsh) + 255) / 256)), dim3(256), 0, st,
+                       logits, n, gsh, lsh, groups, gmax);
+    hipLaunchKernelGGL(choose_topk_kernel, dim3(1), dim3(kThreads), 0, st, logits, n, gsh, groups, gmax, prm,
+                       call ? *call : SampleParams{}, out, tokens, pos);
     return MXH_OK;
 }
 
