@@ -942,6 +942,11 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
+uint8_t* gemm_partials(size_t* bytes) {
+    *bytes = kPartBytes;
+    return reinterpret_cast<uint8_t*>(g_part_ptr);
+}
+
 int gemm_workspace_init() {
     void *p = nullptr, *q = nullptr;
     if (int rc = check_hip(hipGetSymbolAddress(&p, HIP_SYMBOL(g_partials)), "hipGetSymbolAddress(partials)")) return rc;

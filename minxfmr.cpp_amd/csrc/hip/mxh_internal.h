@@ -126,6 +126,8 @@ int gemm_bf16_run(int type, const uint16_t* a, const uint16_t* a_lo, int lda, co
 // workspace is static device memory (gemm_workspace_init, once per process):
 // calls run on the library stream.
 int gemm_workspace_init();
+// its part for partial sums, which other kernels on the library stream may use between GEMMs
+uint8_t* gemm_partials(size_t* bytes);
 bool gemm_q_f16_supported(int type, int k);
 int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda, const uint16_t* s_hi,
                    const uint16_t* s_lo, int lds, const float* rscale, const void* w, float* out, int ldo,

@@ -1,23 +1,30 @@
 // mxh_prefill_attn.hip — causal attention of a chunk of prompt tokens on the
-// fp16 matrix cores, in flash form (running max and sum per query, no score
-// matrix in memory).
+// fp16 matrix cores, in flash form (running reference and sum per query, no
+// score matrix in memory).
 //
 // Reference op: the attention of transformer.cpp:529-629 for each prompt
 // token (scores q.k / sqrt(hd) over cache positions 0 .. pos, softmax
 // softmax.cpp:4-18, weighted sum of V rows), with the chunk's own K/V rows
 // already appended to the fp16 cache by qkv_prep_rows_kernel.
 //
-// Workgroup (g, y) serves kv head g and 64 query rows: the `group` q heads
+// Workgroup (g, y, z) serves kv head g and 64 query rows: the `group` q heads
 // of g for T = 64 / group consecutive tokens (row r = token r / group, head
-// r % group).  Keys stream through LDS in stages of 64, double-buffered.
-// Wave w of four takes query rows 32 (w & 1) .. +32 and key half w >> 1 of
-// every stage; the two waves of a query set see disjoint keys and merge
-// their (max, sum, V sum) at the end.  Per 32-key block a wave computes
+// r % group), over split z of the keys.  Keys stream through LDS in stages of
+// 64, double-buffered.  Wave w of four takes query rows 32 (w & 1) .. +32 and
+// key half w >> 1 of every stage; the two waves of a query set see disjoint
+// keys and merge their (reference, sum, V sum) at the end, the splits of a
+// tile in a second kernel.  Per 32-key block a wave computes
 //
 //   S^T = K Q^T      v_mfma_f32_32x32x16_f16; q is pre-scaled by
 //                    log2(e) / sqrt(hd) and split into fp16 hi + lo (about
 //                    22 significant bits); K is exact (the cache is fp16)
-//   O^T += V^T P^T   P = exp2(S - max) split into fp16 hi + lo; V exact
+//   O^T += V^T P^T   P = 2^(S - ref + 6) split into fp16 hi + lo; V exact
+//
+// ref is the row's largest score when it was last set: it moves (and the sums
+// are rescaled) only where a score exceeds it by more than 8, which is exact
+// and rare.  The 2^6 keeps the low halves of small probabilities out of the
+// fp16 subnormals (2 queries at 7000 against float64: 9.5e-7 without, 5.6e-7
+// with), and P stays below 2^14.
 //
 // Lane l owns query l % 32 in both products (accumulator register i of lane l
 // is row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32), so the softmax
@@ -30,8 +37,18 @@
 // LDS per stage: K as [64 keys][hd] with the 16-byte pieces of a row rotated
 // by an XOR of the key (conflict-free first-product reads), and V transposed
 // as [hd][64 + 8 keys] (a lane's 8 keys contiguous; the 144-byte row stride
-// spreads 16 rows over all banks).  The next stage's global loads are in
-// flight during the current stage's products.
+// spreads 16 rows over all banks; no bank conflicts measured).  The next
+// stage's global loads are in flight during the current stage's products.
+//
+// Bound: a block's 32 MFMAs (1,024 cycles at head dim 128) and its softmax
+// (165 vector instructions, about 850 cycles) follow each other in a wave, and
+// the two waves of a SIMD keep in step, so their times add up (counters at 512
+// queries at 7680: matrix cores busy 43%, vector ALU 50%).  So the vector work
+// was cut: the reference that seldom moves, one-instruction splits, loads
+// without masks.  228 -> 156 us there; the first product one block ahead needs
+// more registers than there are (spills, 258 us), wave priorities change
+// nothing.  Few queries at long positions were a few workgroups' serial walk
+// over the keys: they split them (see the launch).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -42,15 +59,25 @@ namespace mxh {
 
 namespace {
 
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPaRows = 64;        // query rows per workgroup
+constexpr float kPaBias = 6.f, kPaSlack = 8.f;  // P at most 2^(bias + slack)
+
 constexpr int kPaKeys = 64;        // keys per stage
+constexpr int kPaThreads = 256;
 constexpr int kPaVst = kPaKeys + 8;  // transposed V row stride (halves)
 
 __host__ __device__ constexpr int pa_stage_halves(int hd) { return kPaKeys * hd + hd * kPaVst; }
-__host__ __device__ constexpr size_t pa_lds_bytes(int hd) { return (size_t)2 * pa_stage_halves(hd) * 2; }
+// floats a wave leaves for the merge: V sums [hd][32], references, sums
+__host__ __device__ constexpr int pa_merge_floats(int hd) { return hd * 32 + 64; }
+__host__ __device__ constexpr size_t pa_lds_bytes(int hd) {
+    const size_t st = (size_t)2 * pa_stage_halves(hd) * 2, mg = (size_t)4 * pa_merge_floats(hd) * 4;
+    return st > mg ? st : mg;
+}
 
 // row m of a 32-key block -> key (bits 2 and 3 swapped)
 __device__ __forceinline__ int pa_pi(int m) { return (m & ~12) | ((m & 4) << 1) | ((m & 8) >> 1); }
@@ -61,27 +88,52 @@ __device__ __forceinline__ int pa_swz(int key) {
     return (key >> RS) & (NCH - 1);
 }
 
+// the larger / the sum of a value in lanes l and l ^ 32, in both
+__device__ __forceinline__ float pa_pair_max(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// p - h[HALF] in one instruction (written as C++ it is a conversion and a
+// subtraction; exact)
+template <int HALF>
+__device__ __forceinline__ float pa_rest(float p, f16x2 h) {
+    float d;
+    if constexpr (HALF) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h), "v"(p));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h), "v"(p));
+    return d;
+}
+
+// One split's part of one row: V sums part[p][row][hd] and (reference, sum)
+// ml[p][row], p = (tile nkv + g) splits + z
 template <int HD>
-__global__ __launch_bounds__(256) void attention_rows_mfma_kernel(const float* __restrict__ q,
-                                                                  const __half* __restrict__ kc,
-                                                                  const __half* __restrict__ vc,
-                                                                  float* __restrict__ att, int p0, int m, int nh,
-                                                                  int nkv, float qscale) {
+__global__ __launch_bounds__(kPaThreads, 2) void attention_rows_mfma_kernel(
+    const float* __restrict__ q, const __half* __restrict__ kc, const __half* __restrict__ vc,
+    float* __restrict__ att, float* __restrict__ part, float2* __restrict__ ml, int p0, int m, int nh, int nkv,
+    float qscale, int split_stages) {
     constexpr int NCH = HD / 8, KS = HD / 16, DB = HD / 32;
-    constexpr int NKL = kPaKeys * NCH / 256;  // K pieces per thread per stage
-    constexpr int NVB = 16 * NCH;             // 4-key x 8-dim V blocks per stage
+    constexpr int NKL = kPaKeys * NCH / kPaThreads;  // K pieces per thread per stage
+    constexpr int NVB = kPaKeys / 4 * NCH;           // 4-key x 8-dim V blocks per stage
+    static_assert(NKL * kPaThreads == kPaKeys * NCH && NVB <= kPaThreads, "");
     extern __shared__ __align__(16) _Float16 pa_smem[];
 
     const int g = blockIdx.x, group = nh / nkv, T = kPaRows / group;
-    const int t0 = blockIdx.y * T;
+    const int tile = gridDim.y - 1 - blockIdx.y;  // the tiles with the most keys start first
+    const int t0 = tile * T;
     const int kvd = nkv * HD, qd = nh * HD;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qg = wave & 1, kh = wave >> 1, n = lane & 31, h = lane >> 5;
 
     const int tmax = min(t0 + T, m) - 1;
-    const int kend = p0 + tmax + 1;             // keys [0, kend) for the workgroup
+    const int kend = p0 + tmax + 1;             // keys [0, kend) for the tile
     const int lim_min = p0 + t0 + 1;            // smallest per-row limit
-    const int nst = (kend + kPaKeys - 1) / kPaKeys;
+    const int st0 = blockIdx.z * split_stages;
+    const int nst = min((kend + kPaKeys - 1) / kPaKeys, st0 + split_stages);
+    const size_t prt = ((size_t)tile * nkv + g) * gridDim.z + blockIdx.z;
+    if (st0 >= nst) {  // no keys of this tile in the split
+        if (tid < kPaRows) ml[prt * kPaRows + tid] = make_float2(-INFINITY, 0.f);
+        return;
+    }
 
     // this lane's query row
     const int r = 32 * qg + n, tl = r / group, hh = r % group, tok = t0 + tl;
@@ -112,57 +164,50 @@ __global__ __launch_bounds__(256) void attention_rows_mfma_kernel(const float* _
         }
     }
 
-    // stage loads: K pieces (key, 16-byte chunk) and V blocks (4 keys x 8 dims)
-    uint4 kraw[NKL], vraw[4];
-    const size_t col = (size_t)g * HD;
-    auto load = [&](int st) {
-        const int k0 = st * kPaKeys;
+    // stage loads: K pieces (key, 16-byte chunk) and V blocks (4 keys x 8
+    // dims); keys past the last repeat it (their scores are masked)
+    u32x4 kraw[NKL], vraw[4];
+    const uint32_t row_b = 2u * (uint32_t)kvd;
+    const int kk = tid / NCH, kcb = 16 * (tid % NCH);
+    const int vk = 4 * (tid & 15), vcol = tid >> 4;
+    const auto load = [&](int st) __attribute__((always_inline)) {
+        const int last = kend - 1 - st * kPaKeys;  // (uniform)
+        const size_t at = ((size_t)st * kPaKeys * kvd + (size_t)g * HD) * 2;
+        const uint8_t *ks = reinterpret_cast<const uint8_t*>(kc) + at, *vs = reinterpret_cast<const uint8_t*>(vc) + at;
 #pragma unroll
-        for (int u = 0; u < NKL; ++u) {
-            const int i = tid + 256 * u, key = k0 + i / NCH, c = i % NCH;
-            kraw[u] = key < kend ? *reinterpret_cast<const uint4*>(kc + (size_t)key * kvd + col + 8 * c)
-                                 : make_uint4(0, 0, 0, 0);
-        }
-        if (tid < NVB) {
-            const int kg = tid & 15, c = tid >> 4;
+        for (int u = 0; u < NKL; ++u)
+            kraw[u] = *reinterpret_cast<const u32x4*>(ks + (uint32_t)min(kk + kPaThreads / NCH * u, last) * row_b + kcb);
+        if (NVB == kPaThreads || tid < NVB) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = k0 + 4 * kg + i;
-                vraw[i] = key < kend ? *reinterpret_cast<const uint4*>(vc + (size_t)key * kvd + col + 8 * c)
-                                     : make_uint4(0, 0, 0, 0);
-            }
+            for (int i = 0; i < 4; ++i)
+                vraw[i] = *reinterpret_cast<const u32x4*>(vs + (uint32_t)min(vk + i, last) * row_b + 16 * vcol);
         }
     };
-    auto store = [&](int buf) {
+    const auto store = [&](int buf) __attribute__((always_inline)) {
         _Float16* Ks = pa_smem + buf * pa_stage_halves(HD);
         _Float16* Vt = Ks + kPaKeys * HD;
 #pragma unroll
         for (int u = 0; u < NKL; ++u) {
-            const int i = tid + 256 * u, key = i / NCH, c = i % NCH;
-            *reinterpret_cast<uint4*>(Ks + key * HD + 8 * (c ^ pa_swz<HD>(key))) = kraw[u];
+            const int key = kk + kPaThreads / NCH * u;
+            *reinterpret_cast<u32x4*>(Ks + key * HD + 8 * (tid % NCH ^ pa_swz<HD>(key))) = kraw[u];
         }
-        if (tid < NVB) {
-            const int kg = tid & 15, c = tid >> 4;
-            const uint32_t* w0 = reinterpret_cast<const uint32_t*>(&vraw[0]);
-            const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&vraw[1]);
-            const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&vraw[2]);
-            const uint32_t* w3 = reinterpret_cast<const uint32_t*>(&vraw[3]);
+        if (NVB == kPaThreads || tid < NVB) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int sh = 16 * (e & 1), wi = e >> 1;
-                const uint32_t lo = ((w0[wi] >> sh) & 0xffffu) | (((w1[wi] >> sh) & 0xffffu) << 16);
-                const uint32_t hi = ((w2[wi] >> sh) & 0xffffu) | (((w3[wi] >> sh) & 0xffffu) << 16);
-                *reinterpret_cast<uint2*>(Vt + (8 * c + e) * kPaVst + 4 * kg) = make_uint2(lo, hi);
+                const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;  // the high or the low halves of two words
+                *reinterpret_cast<uint2*>(Vt + (8 * vcol + e) * kPaVst + vk) =
+                    make_uint2(__builtin_amdgcn_perm(vraw[1][e >> 1], vraw[0][e >> 1], sel),
+                               __builtin_amdgcn_perm(vraw[3][e >> 1], vraw[2][e >> 1], sel));
             }
         }
     };
 
-    load(0);
-    store(0);
-    if (nst > 1) load(1);
+    load(st0);
+    store(st0 & 1);
+    if (st0 + 1 < nst) load(st0 + 1);
     __syncthreads();
 
-    float mrun = -INFINITY, lrun = 0.f;
+    float mref = -INFINITY, lrun = 0.f;
     f32x16 o[DB];
 #pragma unroll
     for (int d = 0; d < DB; ++d)
@@ -170,58 +215,68 @@ __global__ __launch_bounds__(256) void attention_rows_mfma_kernel(const float* _
         for (int v = 0; v < 16; ++v) o[d][v] = 0.f;
     const int krow = 32 * kh + pa_pi(n);
 
-    for (int st = 0; st < nst; ++st) {
+    for (int st = st0; st < nst; ++st) {
         const _Float16* Ks = pa_smem + (st & 1) * pa_stage_halves(HD);
         const _Float16* Vt = Ks + kPaKeys * HD;
-        f32x16 s;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s[v] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const f16x8 a =
-                *reinterpret_cast<const f16x8*>(Ks + krow * HD + 8 * ((2 * ks + h) ^ pa_swz<HD>(krow)));
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qh[ks], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[ks], s, 0, 0, 0);
-        }
         const int kb = st * kPaKeys + 32 * kh;  // first key of this wave's block
-        if (kb + 31 >= lim_min) {
+        if (kb < kend) {
+            f32x16 s;
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                if (kb + 16 * (v >> 3) + 8 * h + (v & 7) >= lim) s[v] = -INFINITY;
-        }
-        float mx = s[0];
+            for (int v = 0; v < 16; ++v) s[v] = 0.f;
 #pragma unroll
-        for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float mnew = fmaxf(mrun, mx);
-        const float mref = mnew == -INFINITY ? 0.f : mnew;  // a block with every key masked so far
-        const float alpha = __builtin_amdgcn_exp2f(mrun - mref);
-        mrun = mnew;
-        float p[16], ps = 0.f;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            p[v] = __builtin_amdgcn_exp2f(s[v] - mref);
-            ps += p[v];
-        }
-        lrun = lrun * alpha + ps;
-#pragma unroll
-        for (int d = 0; d < DB; ++d)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            f16x8 bh, bl;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const _Float16 hi = (_Float16)p[8 * t + u];
-                bh[u] = hi;
-                bl[u] = (_Float16)(p[8 * t + u] - (float)hi);
+            for (int ks = 0; ks < KS; ++ks) {
+                const f16x8 a =
+                    *reinterpret_cast<const f16x8*>(Ks + krow * HD + 8 * ((2 * ks + h) ^ pa_swz<HD>(krow)));
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qh[ks], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[ks], s, 0, 0, 0);
             }
+            if (kb + 31 >= lim_min) {
 #pragma unroll
-            for (int d = 0; d < DB; ++d) {
-                const f16x8 a = *reinterpret_cast<const f16x8*>(Vt + (32 * d + n) * kPaVst + 32 * kh + 16 * t + 8 * h);
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bh, o[d], 0, 0, 0);
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bl, o[d], 0, 0, 0);
+                for (int v = 0; v < 16; ++v)
+                    if (kb + 16 * (v >> 3) + 8 * h + (v & 7) >= lim) s[v] = -INFINITY;
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+            mx = pa_pair_max(mx);
+            if (__any(mx > mref + kPaSlack)) {  // also the first block with an unmasked key
+                const float mnew = fmaxf(mref, mx);
+                // (every key masked so far: the sums are zero)
+                const float alpha = mref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mref - mnew);
+                mref = mnew;
+                lrun *= alpha;
+#pragma unroll
+                for (int d = 0; d < DB; ++d)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+            }
+            const float bias = mref == -INFINITY ? 0.f : kPaBias - mref;
+            float p[16], ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                p[v] = __builtin_amdgcn_exp2f(s[v] + bias);
+                ps[v & 3] += p[v];
+            }
+            lrun += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                f16x8 bh, bl;
+#pragma unroll
+                for (int u = 0; u < 8; u += 2) {
+                    // hi rounded toward zero, lo what is left: 21 bits at least
+                    const float p0v = p[8 * t + u], p1v = p[8 * t + u + 1];
+                    const f16x2 hi = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(p0v, p1v));
+                    const f16x2 lo = __builtin_bit_cast(
+                        f16x2, __builtin_amdgcn_cvt_pkrtz(pa_rest<0>(p0v, hi), pa_rest<1>(p1v, hi)));
+                    bh[u] = hi[0], bh[u + 1] = hi[1], bl[u] = lo[0], bl[u + 1] = lo[1];
+                }
+#pragma unroll
+                for (int d = 0; d < DB; ++d) {
+                    const f16x8 a =
+                        *reinterpret_cast<const f16x8*>(Vt + (32 * d + n) * kPaVst + 32 * kh + 16 * t + 8 * h);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bh, o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bl, o[d], 0, 0, 0);
+                }
             }
         }
         if (st + 1 < nst) store((st + 1) & 1);
@@ -231,39 +286,110 @@ __global__ __launch_bounds__(256) void attention_rows_mfma_kernel(const float* _
 
     // merge the two key halves of each query set (stage buffers are free now)
     const float lsum = lrun + __shfl_xor(lrun, 32, 64);
-    float* mb = reinterpret_cast<float*>(pa_smem) + qg * (HD * 32 + 64);
-    if (kh == 1) {
+    float* ms = reinterpret_cast<float*>(pa_smem);
+    {
+        float* mb = ms + wave * pa_merge_floats(HD);
 #pragma unroll
         for (int d = 0; d < DB; ++d)
 #pragma unroll
             for (int v = 0; v < 16; ++v) mb[(32 * d + 8 * (v >> 2) + 4 * h + (v & 3)) * 32 + n] = o[d][v];
         if (h == 0) {
-            mb[HD * 32 + n] = mrun;
+            mb[HD * 32 + n] = mref;
             mb[HD * 32 + 32 + n] = lsum;
         }
     }
     __syncthreads();
-    if (kh == 0 && valid) {
-        const float m1 = mb[HD * 32 + n], l1 = mb[HD * 32 + 32 + n];
-        const float M = fmaxf(mrun, m1);  // mrun is finite: key 0 is in this wave's first block
-        const float a0 = __builtin_amdgcn_exp2f(mrun - M), a1 = __builtin_amdgcn_exp2f(m1 - M);
-        const float inv = 1.0f / (a0 * lsum + a1 * l1);
-        float* op = att + (size_t)tok * qd + (size_t)(g * group + hh) * HD;
+    // thread: row 32 mq + mn, dims d0 .. d0 + ND
+    constexpr int ND = HD / 4;
+    const int mq = tid >> 7, mn = tid & 31, d0 = ((tid >> 5) & 3) * ND;
+    const float* mb[2];
+    float a[2], M = -INFINITY, L = 0.f;
 #pragma unroll
-        for (int d = 0; d < DB; ++d)
+    for (int i = 0; i < 2; ++i) {
+        mb[i] = ms + (2 * i + mq) * pa_merge_floats(HD);
+        M = fmaxf(M, mb[i][HD * 32 + mn]);
+    }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int dim = 32 * d + 8 * i + 4 * h;
-                float4 w;
-                w.x = (a0 * o[d][4 * i + 0] + a1 * mb[(dim + 0) * 32 + n]) * inv;
-                w.y = (a0 * o[d][4 * i + 1] + a1 * mb[(dim + 1) * 32 + n]) * inv;
-                w.z = (a0 * o[d][4 * i + 2] + a1 * mb[(dim + 2) * 32 + n]) * inv;
-                w.w = (a0 * o[d][4 * i + 3] + a1 * mb[(dim + 3) * 32 + n]) * inv;
-                *reinterpret_cast<float4*>(op + dim) = w;
-            }
+    for (int i = 0; i < 2; ++i) {
+        const float mi = mb[i][HD * 32 + mn];
+        a[i] = mi == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mi - M);  // (no key of the row in that half)
+        L += a[i] * mb[i][HD * 32 + 32 + mn];
+    }
+    const int row = 32 * mq + mn, mtok = t0 + row / group;
+    float* op;
+    float inv = 1.f;
+    if (gridDim.z > 1) {
+        op = part + (prt * kPaRows + row) * HD;
+        if (d0 == 0) ml[prt * kPaRows + row] = make_float2(M, L);
+    } else {
+        if (row >= T * group || mtok >= m) return;
+        op = att + (size_t)mtok * qd + (size_t)(g * group + row % group) * HD;
+        inv = 1.0f / L;
+    }
+#pragma unroll
+    for (int d = 0; d < ND; d += 4) {
+        float w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int at = (d0 + d + e) * 32 + mn;
+            w[e] = (a[0] * mb[0][at] + a[1] * mb[1][at]) * inv;
+        }
+        *reinterpret_cast<float4*>(op + d0 + d) = make_float4(w[0], w[1], w[2], w[3]);
     }
 }
 
+// att from the splits' parts; a thread takes four dims of one row
+template <int HD>
+__global__ __launch_bounds__(256) void attention_rows_merge_kernel(const float* __restrict__ part,
+                                                                   const float2* __restrict__ ml,
+                                                                   float* __restrict__ att, int m, int nh, int nkv,
+                                                                   int splits, int rows) {
+    const int u = blockIdx.x * 256 + threadIdx.x, d = 4 * (u % (HD / 4)), wr = u / (HD / 4);  // row of all tiles
+    if (wr >= rows) return;
+    const int group = nh / nkv, T = kPaRows / group, row = wr % kPaRows, wg = wr / kPaRows;
+    const int g = wg % nkv, tok = wg / nkv * T + row / group;
+    if (row >= T * group || tok >= m) return;
+    const size_t p = (size_t)wg * splits;
+    float M = -INFINITY, L = 0.f;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr int kAhead = 8;  // splits whose loads are in flight together
+    for (int z0 = 0; z0 < splits; z0 += kAhead) {
+        float2 t[kAhead];
+        float4 v[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const size_t at = (p + min(z0 + i, splits - 1)) * kPaRows + row;
+            t[i] = ml[at];
+            v[i] = *reinterpret_cast<const float4*>(part + at * HD + d);
+        }
+        float m1 = M;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) m1 = fmaxf(m1, t[i].x);
+        const float a0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m1);  // (split 0 holds key 0: m1 is finite)
+        M = m1;
+        L *= a0, s.x *= a0, s.y *= a0, s.z *= a0, s.w *= a0;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            if (z0 + i >= splits || t[i].x == -INFINITY) continue;  // no key of the row in that split
+            const float a = __builtin_amdgcn_exp2f(t[i].x - M);
+            L += a * t[i].y;
+            s.x += a * v[i].x, s.y += a * v[i].y, s.z += a * v[i].z, s.w += a * v[i].w;
+        }
+    }
+    const float inv = 1.0f / L;
+    *reinterpret_cast<float4*>(att + (size_t)tok * nh * HD + (size_t)(g * group + row % group) * HD + d) =
+        make_float4(s.x * inv, s.y * inv, s.z * inv, s.w * inv);
+}
+
+// Splits of the keys among workgroups.  Measured: a stage takes kStage us
+// alone (latencies) and at least kFull us of a CU's time for each workgroup on
+// it, and kSlots workgroups fit a CU; a merge costs its launch (3.5 us), a
+// little a split, and the parts' way through memory.  us without splits / with
+// the splits chosen (m at p0, q heads / kv heads x head dim):
+//   16 at 7680, 32/8 x 128   146 / 22      2 at 7000, 8/1 x 64     90 / 13
+//   128 at 4000, 32/8 x 128   85 / 37      100 at 3000, 8/1 x 32   36 / 12
+//   512 at 7680, 32/8 x 128  210 / 183     512 at 7680, 16/8 x 64 115 / 56
+constexpr int kPaSplitsMax = 32;
 template <int HD>
 int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half* vc, float* att, int p0, int m,
                                   int nh, int nkv, float qscale, hipStream_t st) {
@@ -274,10 +400,35 @@ int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half
             return MXH_ERR_HIP;
         attr_set = true;
     }
-    const int T = kPaRows / (nh / nkv);
-    const dim3 grid((unsigned)nkv, (unsigned)((m + T - 1) / T));
-    hipLaunchKernelGGL(attention_rows_mfma_kernel<HD>, grid, dim3(256), pa_lds_bytes(HD), st, q, kc, vc, att, p0, m,
-                       nh, nkv, qscale);
+    constexpr double kStart = 4.0, kStage = HD == 128 ? 1.45 : HD == 64 ? 0.85 : 0.7;
+    constexpr double kFull = HD == 128 ? 1.3 : HD == 64 ? 0.75 : 0.5;
+    constexpr int kCus = 256, kSlots = HD == 128 ? 2 : HD == 64 ? 3 : 4;
+    const int T = kPaRows / (nh / nkv), tiles = (m + T - 1) / T;
+    const int64_t wgs = (int64_t)nkv * tiles;
+    const int stages = (int)(((int64_t)p0 + m + kPaKeys - 1) / kPaKeys);
+    size_t part_bytes = 0;
+    float* part = reinterpret_cast<float*>(gemm_partials(&part_bytes));
+    int splits = 1, per = stages;
+    double best = 1e30;
+    for (int s = 1; s <= kPaSplitsMax && s <= stages; ++s) {
+        const size_t bytes = (size_t)wgs * s * kPaRows * (HD + 2) * 4;
+        if (s > 1 && bytes > part_bytes) break;
+        const int p = (stages + s - 1) / s;
+        if ((stages + p - 1) / p != s) continue;  // the same stages in fewer splits
+        const int64_t on_cu = (wgs * s + kCus - 1) / kCus, rounds = (on_cu + kSlots - 1) / kSlots;
+        const double full = kFull * (double)on_cu, alone = kStage * (double)rounds;
+        double us = kStart * (double)rounds + p * (full > alone ? full : alone);
+        if (s > 1) us += 3.5 + 0.3 * s + (double)bytes / 5e6;
+        if (us < best) best = us, splits = s, per = p;
+    }
+    float2* ml = reinterpret_cast<float2*>(part + (size_t)wgs * splits * kPaRows * HD);  // (splits > 1)
+    hipLaunchKernelGGL(attention_rows_mfma_kernel<HD>, dim3((unsigned)nkv, (unsigned)tiles, (unsigned)splits),
+                       dim3(kPaThreads), pa_lds_bytes(HD), st, q, kc, vc, att, part, ml, p0, m, nh, nkv, qscale, per);
+    if (splits > 1) {
+        const int rows = (int)wgs * kPaRows;
+        hipLaunchKernelGGL(attention_rows_merge_kernel<HD>, dim3((unsigned)((rows * (HD / 4) + 255) / 256)), dim3(256),
+                           0, st, part, ml, att, m, nh, nkv, splits, rows);
+    }
     return MXH_OK;
 }
 

@@ -1,0 +1,47 @@
+"""Prefill attention where the keys are split among workgroups, and where the
+running reference moves (GPU).
+
+Few query tiles over many keys split the keys; parts of a tile may hold no key
+of a row, or none of the tile (causal chunks from position 0).  Expected values
+and the admitted error as in test_attention_prefill_gpu.py.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import mxhip
+from test_attention_prefill_gpu import reference
+
+pytestmark = pytest.mark.gpu
+
+# (nh, nkv, hd, p0, m): one query, a partial tile, odd groups, splits that end
+# inside the chunk, tiles with fewer keys than the others
+CASES = [(8, 1, 64, 2000, 1), (32, 8, 128, 1500, 16), (7, 1, 128, 640, 9), (3, 1, 32, 1023, 2), (8, 1, 128, 0, 300),
+         (4, 4, 64, 0, 513), (14, 2, 64, 191, 65), (8, 8, 32, 64, 64)]
+
+
+@pytest.mark.parametrize("kind", ["flat", "rising"])
+@pytest.mark.parametrize("nh,nkv,hd,p0,m", CASES, ids=[f"h{a}-kv{b}-d{c}-p{d}-m{e}" for a, b, c, d, e in CASES])
+def test_attention_splits(mxh, nh, nkv, hd, p0, m, kind):
+    rng = np.random.default_rng(nh * 1000 + hd * 10 + p0 + m)
+    n_ctx = p0 + m + 40
+    q = rng.standard_normal((m, nh * hd)).astype(np.float32)
+    kc = rng.standard_normal((n_ctx, nkv * hd)).astype(np.float16)
+    if kind == "rising":  # scores grow with the key's position, by many powers of two over the row
+        q = np.abs(q) * np.float32(0.5)
+        kc = np.abs(kc) * np.linspace(0.0, 4.0, n_ctx, dtype=np.float16)[:, None]
+    vc = rng.standard_normal((n_ctx, nkv * hd)).astype(np.float16)
+    kc[p0 + m:] = np.float16(np.nan)
+    vc[p0 + m:] = np.float16(np.nan)
+    dq, dk, dv = (mxhip.DeviceBuffer.from_array(a) for a in (q, kc, vc))
+    att = mxhip.DeviceBuffer.from_array(np.full(m * nh * hd, np.nan, np.float32))
+    mxhip.attention_prefill(dq, dk, dv, att, p0, m, nh, nkv, hd)
+    got = att.download(np.float32, m * nh * hd).reshape(m, nh * hd).astype(np.float64)
+    want = reference(q, kc, vc, p0, m, nh, nkv, hd)
+    bound = 1e-4 * float(np.abs(vc[: p0 + m].astype(np.float64)).max()) + 1e-4 * np.abs(want)
+    err = np.abs(got - want)
+    assert np.all(np.isfinite(got)), "non-finite output"
+    assert np.all(err <= bound), f"worst {float((err / bound).max()):.3g} x bound"
+    for b in (dq, dk, dv, att):
+        b.close()
