@@ -122,7 +122,9 @@ int mxh_gemv(int type, const void *w, const float *x, float *y, int64_t n, int64
  * CUDA backend uploads (cuda_backend.cu:364-394). */
 int mxh_tile_rows(int type, void *w, int64_t rows, int64_t cols, int *tiled);
 
-/* out[m x n] = A[m x k] . dequant(W[n x k])^T for any m (prefill).
+/* out[m x n] = A[m x k] . dequant(W[n x k])^T for any m, in mxh_gemv's
+ * arithmetic (the same bits as one mxh_gemv per row), several rows per pass
+ * over the weights.
  * Replaces backend_matmul_rhs_transposed (src/backend/backend_runtime.h:37). */
 int mxh_matmul_rhs_t(int type, const float *a, int64_t m, const void *w, int64_t n, int64_t k, float *out,
                      int form);
