@@ -17,7 +17,7 @@
 // Bound: the one workgroup's chain of barriers and LDS latencies, two launches
 // and the wait for the id.  Selecting by sorting (64 lists sorted in LDS, then
 // 4,096 keys by one workgroup) took 156 us for top_k 40 of 151,936 ids with
-// the copies of its parameters and of the id; this 34.
+// the copies of its parameters and of the id; this 27.
 //
 // The uniform of draw d is splitmix64 at state seed + (d + 1) *
 // 0x9E3779B97F4A7C15, the d-th value of the sequence that starts at `seed`.
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
     __shared__ __attribute__((aligned(16))) uint16_t list[kGroupsMax];  // groups taken, then the ids in order
     __shared__ int part[2][4][kWaves];
     __shared__ int n_list, n_cand;
-    __shared__ uint32_t top;
+    __shared__ uint32_t bound;
     static_assert(sizeof(list) >= kCandMax * sizeof(int) && kGroupsMax <= 65536, "");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const SampleParams sp = prm ? *prm : call;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
         mx[r] = g < groups ? gmax[g] : 0u;
         my_top = max(my_top, mx[r]);
     }
-    if (tid == 0) n_list = 0, n_cand = 0, top = 0u;
+    if (tid == 0) n_list = 0, n_cand = 0, bound = 0u;
     // per-wave counts -> the workgroup's (part is double-buffered: one barrier a call)
     int turn = 0;
     const auto total3 = [&](int a, int b, int c, int (&t)[3]) {
@@ -248,9 +248,34 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
     };
 
     // T: the k-th largest group maximum, from the top bit down, or a value
-    // below it that few more maxima reach; 0 (every key) with fewer groups
+    // below it that few more maxima reach; 0 (every key) with fewer groups.
+    // For k up to a quarter of the threads the largest maximum of each thread
+    // stands for its groups (hardly more keys reach the k-th of those) and one
+    // wave searches, without barriers: 2.4 us against 7.4.
     uint32_t T = 0u;
-    if (groups >= k)
+    if (k <= kThreads / 4) {
+        uint32_t* tops = reinterpret_cast<uint32_t*>(s);
+        tops[tid] = my_top;
+        __syncthreads();
+        if (wave == 0) {
+            uint32_t v[kWaves];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) v[w] = tops[lane + 64 * w];
+            for (int bit = 31; bit >= 0; --bit) {
+                const uint32_t c = T | (1u << bit);
+                int t = 0;
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) t += __popcll(__ballot(v[w] >= c));
+                if (t >= k) {
+                    T = c;
+                    if (t <= k + (k >> 3)) break;
+                }
+            }
+            if (lane == 0) bound = T;
+        }
+        __syncthreads();
+        T = bound;
+    } else if (groups >= k) {
         for (int bit = 31; bit >= 0; --bit) {
             const uint32_t c = T | (1u << bit);
             int cnt = 0;
@@ -267,21 +292,30 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
                 if (t <= k + (k >> 3)) break;
             }
         }
+    }
     __syncthreads();
 
-    // the groups whose maximum reaches T
+    // the groups whose maximum reaches T; one place a wave in the list
+    {
+        uint64_t in[kGroupRegs];
+        int n_in = 0;
 #pragma unroll
-    for (int r = 0; r < kGroupRegs; ++r) {
-        const int g = tid + kThreads * r;
-        const bool in = g < groups && mx[r] >= T;
-        const uint64_t mask = __ballot(in);
-        if (!mask) continue;
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&n_list, __popcll(mask));
-        base = __builtin_amdgcn_readfirstlane(base);
-        if (in) list[base + __popcll(mask & ((1ull << lane) - 1))] = (uint16_t)g;
+        for (int r = 0; r < kGroupRegs; ++r) {
+            in[r] = __ballot(tid + kThreads * r < groups && mx[r] >= T);
+            n_in += __popcll(in[r]);
+        }
+        if (n_in) {
+            int base = 0;
+            if (lane == 0) base = atomicAdd(&n_list, n_in);
+            base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+            for (int r = 0; r < kGroupRegs; ++r) {
+                if (in[r] >> lane & 1)
+                    list[base + __popcll(in[r] & ((1ull << lane) - 1))] = (uint16_t)(tid + kThreads * r);
+                base += __popcll(in[r]);
+            }
+        }
     }
-    atomicMax(&top, my_top);
     __syncthreads();
 
     // f(key, valid) over their ids, whole waves at a time
@@ -310,6 +344,11 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
         // The k-th largest key, or one below it that at most kCandMax reach:
         // two bits a pass.  It lies between T and the largest maximum, so the
         // value bits above their first difference are known; then the id's.
+        if (tid == 0) bound = 0u;
+        __syncthreads();
+        atomicMax(&bound, my_top);
+        __syncthreads();
+        const uint32_t top = bound;
         int id_bits = 1;
         while (id_bits < 31 && (n >> id_bits)) ++id_bits;
         const uint32_t diff = T ^ top;
