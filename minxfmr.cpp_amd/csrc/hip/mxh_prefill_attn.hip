@@ -21,8 +21,8 @@
 //   O^T += V^T P^T   P = 2^(S - ref + 6) split into fp16 hi + lo; V exact
 //
 // ref is the row's largest score when it was last set: it moves (and the sums
-// are rescaled) only where a score exceeds it by more than 8, which is exact
-// and rare.  The 2^6 keeps the low halves of small probabilities out of the
+// are rescaled, all by one rounded factor) only where a score exceeds it by
+// more than 8, which is rare.  The 2^6 keeps the low halves of small probabilities out of the
 // fp16 subnormals (2 queries at 7000 against float64: 9.5e-7 without, 5.6e-7
 // with), and P stays below 2^14.
 //
@@ -61,6 +61,7 @@ namespace {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -263,11 +264,12 @@ __global__ __launch_bounds__(kPaThreads, 2) void attention_rows_mfma_kernel(
                 f16x8 bh, bl;
 #pragma unroll
                 for (int u = 0; u < 8; u += 2) {
-                    // hi rounded toward zero, lo what is left: 21 bits at least
+                    // both halves rounded to nearest (one instruction for two): no mean error.
+                    // Cut off, they leave the V sums 7e-8 to 9e-8 low against lrun.
                     const float p0v = p[8 * t + u], p1v = p[8 * t + u + 1];
-                    const f16x2 hi = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(p0v, p1v));
-                    const f16x2 lo = __builtin_bit_cast(
-                        f16x2, __builtin_amdgcn_cvt_pkrtz(pa_rest<0>(p0v, hi), pa_rest<1>(p1v, hi)));
+                    const f16x2 hi = __builtin_convertvector((f32x2{p0v, p1v}), f16x2);
+                    const f16x2 lo =
+                        __builtin_convertvector((f32x2{pa_rest<0>(p0v, hi), pa_rest<1>(p1v, hi)}), f16x2);
                     bh[u] = hi[0], bh[u + 1] = hi[1], bl[u] = lo[0], bl[u + 1] = lo[1];
                 }
 #pragma unroll

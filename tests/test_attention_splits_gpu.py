@@ -45,3 +45,26 @@ def test_attention_splits(mxh, nh, nkv, hd, p0, m, kind):
     assert np.all(err <= bound), f"worst {float((err / bound).max()):.3g} x bound"
     for b in (dq, dk, dv, att):
         b.close()
+
+
+@pytest.mark.parametrize("nh,nkv,hd,p0,m", [(8, 2, 128, 200, 256), (8, 8, 64, 900, 256), (4, 1, 32, 3000, 64)],
+                         ids=["whole", "d64", "split"])
+def test_attention_probabilities_are_unbiased(mxh, nh, nkv, hd, p0, m):
+    """With every V element 1 the outputs are sum(hi + lo of P) / sum(P): the
+    split's own error.  Two halves rounded to nearest leave no mean error (a
+    few 1e-9 over these rows, from the fp32 sums); a low half cut off instead
+    lacks half a unit of its last place on average, with one sign: of P in
+    [1, 2) that is 4/3 2^-23, -1.1e-7 at most.  2^-25 (3e-8) lies between.
+    """
+    rng = np.random.default_rng(hd + p0)
+    q = rng.standard_normal((m, nh * hd)).astype(np.float32)
+    kc = rng.standard_normal((p0 + m, nkv * hd)).astype(np.float16)
+    vc = np.ones((p0 + m, nkv * hd), np.float16)
+    dq, dk, dv = (mxhip.DeviceBuffer.from_array(a) for a in (q, kc, vc))
+    att = mxhip.DeviceBuffer(4 * m * nh * hd)
+    mxhip.attention_prefill(dq, dk, dv, att, p0, m, nh, nkv, hd)
+    err = att.download(np.float32, m * nh * hd).astype(np.float64) - 1.0
+    assert np.abs(err).max() <= 1e-6, f"worst {np.abs(err).max():.3g}"
+    assert abs(err.mean()) <= 2.0 ** -25, f"mean error {err.mean():.3g}"
+    for b in (dq, dk, dv, att):
+        b.close()
