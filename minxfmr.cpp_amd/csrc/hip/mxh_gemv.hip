@@ -1314,10 +1314,17 @@ __device__ __forceinline__ void stage_rows(float* smem, const float* __restrict_
     __syncthreads();
 }
 
-// dwords of LDS one staged row of x takes
+// dwords of LDS one staged row of x takes: whole 16-byte units, so that every
+// row's 16-byte accesses are aligned (k + k / 16 alone is not where k % 64 is 32)
 template <class Ty, int W>
 __host__ __device__ constexpr int rows_stride(int k) {
-    return Ty::kIntX ? xq_dwords<W>(k) : k + k / 16;
+    return Ty::kIntX ? xq_dwords<W>(k) : (k + k / 16 + 3) & ~3;
+}
+template <class Ty, int W>
+constexpr bool rows_aligned() {
+    for (int k = 32; k <= 15360; k += 32)
+        if (rows_stride<Ty, W>(k) % 4 || (!Ty::kIntX && rows_stride<Ty, W>(k) < k + 4 * ((k - 1) / 64))) return false;
+    return true;
 }
 
 template <template <int> class T, int R, int MB, int W>
@@ -1619,6 +1626,7 @@ constexpr size_t kRowsLds = 160 * 1024;
 
 template <template <int> class T, int R, int MB>
 int rows_launch_mb(const uint8_t* w, const float* x, float* y, int n, int k, int rows, int form, hipStream_t st) {
+    static_assert(rows_aligned<T<R>, kRowsWaves>(), "16-byte LDS accesses of every staged row");
     auto kern = gemv_rows_kernel<T, R, MB, kRowsWaves>;
     static bool attr_set = false;  // above 64 KiB of LDS needs the opt-in, once per kernel
     if (!attr_set) {
