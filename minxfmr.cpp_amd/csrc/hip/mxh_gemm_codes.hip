@@ -10,7 +10,7 @@
 //   Q4_K, Q5_K  w = d sc_j q - dmin m_j: codes sc_j q (< 2048), d per
 //               256-element block; the min terms are a second contraction
 //               over the activations' sub-block sums, eight per block.
-//   Q8_0        w = d q: codes q, d per 32-element block.
+//   Q8_0, Q5_0  w = d q: codes q (Q5_0: q - 16), d per 32-element block.
 //   Q6_K        w = d sc_j (q - 32): sc_j (q - 32) needs 13 bits, so it is a
 //               pair of codes, the fp16 rounding Wh and the exact rest Wl;
 //               d per 256-element block.  Wl . a_lo, below 2^-23 of the
@@ -224,6 +224,36 @@ struct Fmt<GF_Q80T> {
     }
 };
 
+// Q8_0 and Q5_0 rows in GGUF order: eight blocks are 272 (Q8_0) or 176 (Q5_0) bytes, so rows
+// and every eighth block are 16-byte aligned.  A granule of four blocks comes
+// as the 16-byte pieces that hold it, d and all; an odd one starts 8 bytes
+// into its first piece.  Read in place since regrouping them into the tiled
+// order first cost a read and a write of the weights: Q8_0 2 x 30000 x 14336
+// 725 us so, 149 in place; 200 x 24576 x 4096 279 and 142 (tiled rows 127).
+template <int BLOCK>
+struct FmtBlock32 {
+    static constexpr int kH = 0, kGR = 2, kNT = 1, kNC = (4 * BLOCK + 15) / 16, kBlock = BLOCK;
+    static constexpr bool kMin = false, kSplitW = false, kRuns = false, kPair = true;
+    static __host__ __device__ constexpr int slice_chunk(int half, int sl) { return 2 * half + sl; }
+    static __device__ __forceinline__ int type(int) { return 0; }
+    static __device__ __forceinline__ int chunk(int, int p) { return p; }
+    static __device__ __forceinline__ uint32_t q_off(uint32_t gr, uint32_t, uint32_t) {
+        return (gr >> 1) * (8 * BLOCK) + (gr & 1) * (4 * BLOCK - 8);
+    }
+    // byte of block `half` of step g of its 256 elements, in its granule's pieces
+    static __host__ __device__ constexpr int block_at(int g, int half) {
+        return 8 * (g >> 1) + BLOCK * (2 * (g & 1) + half);
+    }
+};
+template <>
+struct Fmt<GF_Q80> : FmtBlock32<34> {
+    static constexpr int kType = MXH_Q8_0, kQL = 10;
+};
+template <>
+struct Fmt<GF_Q50> : FmtBlock32<22> {
+    static constexpr int kType = MXH_Q5_0, kQL = 12;
+};
+
 // a step is a 64-element chunk of the tiled layout: four runs of 16 elements
 // (kRuns: 32 apart), so the activations are staged in that order
 template <>
@@ -289,9 +319,13 @@ struct Geo {
 // operand reads: 8 consecutive rows take 8 different chunk slots)
 __device__ __forceinline__ int a_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
-// XOR of the piece index of weight row `row` in a run of NC pieces
+// XOR of the piece index of weight row `row` in a run of NC pieces (rows of
+// nine or six pieces spread over the banks as they are)
 template <int NC>
-__device__ __forceinline__ int w_swz(int row) { return (row / (16 / NC)) & (NC - 1); }
+__device__ __forceinline__ int w_swz(int row) {
+    if constexpr (NC & (NC - 1)) return 0;
+    else return (row / (16 / NC)) & (NC - 1);
+}
 
 template <int F, int WM, int MI, int NJ, int NST>
 __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
@@ -349,12 +383,13 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     const uint32_t voff_d =
         (uint32_t)(min(n0 + (wave * 64) % BN + lane, a.n - 1) - n0) * (uint32_t)rb;  // (waves past BN / 64 repeat rows)
     // headers, then sub-block sums (hi rows, lo rows)
-    const uint8_t* hptr[G::kHL];
-    int hpiece[G::kHL], hslot[G::kHL];
-    uint32_t is_sum[G::kHL];
+    constexpr int kHA = G::kHL ? G::kHL : 1;
+    const uint8_t* hptr[kHA];
+    int hpiece[kHA], hslot[kHA];
+    uint32_t is_sum[kHA];
 #pragma unroll
     for (int u = 0; u < G::kHL; ++u) {
-        const int s = (u * 512 + wave * 64) % G::kHN;
+        const int s = (u * 512 + wave * 64) % (G::kHN ? G::kHN : 1);
         hslot[u] = s;
         is_sum[u] = s >= FM::kH * BN;
         hpiece[u] = is_sum[u] ? 0 : s / BN;
@@ -385,10 +420,12 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
             const uint32_t hb = lds0 + NST * G::kA + 2 * G::kW + (uint32_t)((st >> 2) & 1) * G::kHdr;
 #pragma unroll
             for (int u = 0; u < G::kHL; ++u) {
-                uint32_t off = FM::h_off(b, hpiece[u], nblk);
-                // (arithmetic, not a branch: the step stays one block of code)
-                if constexpr (FM::kMin) off += (16u * b - off) * is_sum[u];
-                g2l_v(hptr[u] + off, hb + hslot[u] * 16);
+                if constexpr (FM::kH > 0) {
+                    uint32_t off = FM::h_off(b, hpiece[u], nblk);
+                    // (arithmetic, not a branch: the step stays one block of code)
+                    if constexpr (FM::kMin) off += (16u * b - off) * is_sum[u];
+                    g2l_v(hptr[u] + off, hb + hslot[u] * 16);
+                }
             }
             if constexpr (G::kDL) g2l4_s(wbase + FM::d_off(b, nblk), voff_d, hb + G::kHN * 16 + wave * 256);
         }
@@ -442,6 +479,7 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
         }
     };
     auto read_head = [&](int t) __attribute__((always_inline)) {
+        if constexpr (FM::kH == 0) return;
         const uint8_t* hb = hdrs + (size_t)((t >> 2) & 1) * G::kHdr;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -463,14 +501,44 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
     };
     // the raw codes of step t (st: t modulo the granule)
     auto read_q = [&](int t, auto sc) __attribute__((always_inline)) {
-        constexpr int st = decltype(sc)::value % FM::kGR;
+        constexpr int g = decltype(sc)::value, st = g % FM::kGR;
         const uint8_t* wq = codes + (size_t)((t / FM::kGR) & 1) * G::kW;
         auto piece = [&](int j, int p) {
             return wq + (FM::type(p) * (BN * FM::kNC) + col[j] * FM::kNC + (FM::chunk(st, p) ^ w_swz<FM::kNC>(col[j]))) * 16;
         };
+        // dword i of the words at a 4-byte aligned place of the row's pieces
+        auto word = [&](int j, int at, int i) {
+            return *reinterpret_cast<const uint32_t*>(wq + col[j] * (16 * FM::kNC) + at + 4 * i);
+        };
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if constexpr (F == GF_Q6KT) {
+            if constexpr (F == GF_Q80) {
+                // the lane's 16 codes of each block, and its d; the first
+                // block's codes start in the middle of a dword
+                const int b0q = FM::block_at(g, 0) + 16 * hh, b1q = FM::block_at(g, 1) + 2 + 16 * hh;
+                uint32_t w[5];
+#pragma unroll
+                for (int i = 0; i < 5; ++i) w[i] = word(j, b0q, i);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    q[j][i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2);
+                    q[j][4 + i] = word(j, b1q, i);
+                }
+                q[j][8] = word(j, FM::block_at(g, 0), 0);            // d in its low half
+                q[j][9] = word(j, FM::block_at(g, 1) - 2, 0) >> 16;
+            } else if constexpr (F == GF_Q50) {
+                // per block four dwords of nibbles, the high bits, d
+                uint32_t w[6];
+#pragma unroll
+                for (int i = 0; i < 6; ++i) w[i] = word(j, FM::block_at(g, 0), i);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[j][i] = __builtin_amdgcn_alignbyte(w[i + 2], w[i + 1], 2);
+                q[j][4] = __builtin_amdgcn_alignbyte(w[1], w[0], 2);
+                q[j][5] = w[0];
+#pragma unroll
+                for (int i = 0; i < 5; ++i) q[j][6 + i] = word(j, FM::block_at(g, 1) + 2, (i + 1) % 5);
+                q[j][11] = word(j, FM::block_at(g, 1) - 2, 0) >> 16;
+            } else if constexpr (F == GF_Q6KT) {
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
                     const uint2 v = *reinterpret_cast<const uint2*>(piece(j, p) + 8 * hh);
@@ -519,7 +587,25 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
                 }
                 W[half][0][j] = pack8(l[0], l[1], l[2], l[3]);
                 W[half][1][j] = pack8(h[0], h[1], h[2], h[3]);
-            } else if constexpr (F == GF_Q80T) {
+            } else if constexpr (F == GF_Q50) {
+                // this lane half's nibbles and high bits: elements 16 hh .. +15
+                const uint32_t hb = q[j][6 * half + 4] >> (16 * hh);
+                uint32_t o[8];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const uint32_t w0 = q[j][6 * half + x] >> (4 * hh);
+                    // bit e of the four high bits to bits 4 + e and 18 + e
+                    const uint32_t b = ((hb >> (4 * x)) & 15u) * 0x40010u;
+                    const uint32_t c0 = code_pair(b, 0x00100010u, code_pair(w0, 0x000f000fu, kMagic));
+                    const uint32_t c1 = code_pair(b >> 1, 0x00100010u, code_pair(w0 >> 8, 0x000f000fu, kMagic));
+                    const f16x2 off = splat((_Float16)1040.f);
+                    o[2 * x] = as_u(as_h2(c0) - off);
+                    o[2 * x + 1] = as_u(as_h2(c1) - off);
+                }
+                W[half][0][j] = pack8(o[0], o[1], o[2], o[3]);
+                W[half][1][j] = pack8(o[4], o[5], o[6], o[7]);
+                d2[half][j] = half_lo(q[j][6 * half + 5]);
+            } else if constexpr (F == GF_Q80T || F == GF_Q80) {
                 uint32_t o[8];
 #pragma unroll
                 for (int x = 0; x < 4; ++x) {
@@ -530,8 +616,12 @@ __global__ __launch_bounds__(kThreads) void gemm_codes_kernel(CodesArgs a) {
                 }
                 W[half][0][j] = pack8(o[0], o[1], o[2], o[3]);
                 W[half][1][j] = pack8(o[4], o[5], o[6], o[7]);
-                const uint32_t dw = g == 0 ? hd[j].x : g == 1 ? hd[j].y : g == 2 ? hd[j].z : hd[j].w;
-                d2[half][j] = half ? half_hi(dw) : half_lo(dw);
+                if constexpr (F == GF_Q80) {
+                    d2[half][j] = half_lo(q[j][8 + half]);
+                } else {
+                    const uint32_t dw = g == 0 ? hd[j].x : g == 1 ? hd[j].y : g == 2 ? hd[j].z : hd[j].w;
+                    d2[half][j] = half ? half_hi(dw) : half_lo(dw);
+                }
             } else {  // Q6_K: runs r = 2 half, 2 half + 1 (elements 32 r + 16 p + i of the block's half)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
@@ -753,7 +843,9 @@ int gemm_codes_launch(GemmFmt f, GemmTile t, const CodesArgs& a, hipStream_t st)
     case GF_Q4KT: return codes_tile<GF_Q4KT>(t, a, st);
     case GF_Q5K: return codes_tile<GF_Q5K>(t, a, st);
     case GF_Q5KT: return codes_tile<GF_Q5KT>(t, a, st);
+    case GF_Q80: return codes_tile<GF_Q80>(t, a, st);
     case GF_Q80T: return codes_tile<GF_Q80T>(t, a, st);
+    case GF_Q50: return codes_tile<GF_Q50>(t, a, st);
     case GF_Q6KT: return codes_tile<GF_Q6KT>(t, a, st);
     }
     return MXH_ERR_UNSUPPORTED;
@@ -822,73 +914,32 @@ static __device__ __align__(256) uint8_t g_slab[kSlabBytes];
 float* g_part_ptr = nullptr;
 uint8_t* g_slab_ptr = nullptr;
 
-// Rows whose blocks are only 2-aligned, regrouped into the kernel's tiled
-// orders: Q8_0 and Q5_0 (its value d (q - 16) is a Q8_0 block's) as tiled
-// Q8_0, Q6_K as tiled Q6_K with the block count rounded up to a multiple of
-// eight (16-byte rows; the added blocks are never read).  Thread: one 32-element
-// block, or one 64-element Q6_K chunk.  Bound by HBM: reads and writes each
-// byte once.
+// Q6_K rows in GGUF order are only 2-aligned (210-byte blocks): regrouped into
+// the tiled order, the block count rounded up to a multiple of eight (16-byte
+// rows; the added blocks are never read).  Thread: one 64-element chunk.
+// Bound by HBM: reads and writes each byte once.
 __device__ __forceinline__ uint4 ld_u16x8(const uint8_t* p) {
     const uint16_t* h = reinterpret_cast<const uint16_t*>(p);
     return make_uint4(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16), h[4] | ((uint32_t)h[5] << 16),
                       h[6] | ((uint32_t)h[7] << 16));
 }
 
-template <int TYPE>
-__global__ __launch_bounds__(256) void regroup_rows_kernel(const uint8_t* __restrict__ w, uint8_t* __restrict__ o,
-                                                           int rows, int k, int row_blocks) {
-    constexpr int kUnit = TYPE == MXH_Q6_K ? 64 : 32;
-    const int units = k / kUnit;
+__global__ __launch_bounds__(256) void regroup_q6k_kernel(const uint8_t* __restrict__ w, uint8_t* __restrict__ o,
+                                                          int rows, int k, int row_blocks) {
+    const int units = k / 64;
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int row = (int)(t / units), c = (int)(t % units);
     if (row >= rows) return;
-    const uint8_t* rp = w + (size_t)row * row_bytes(TYPE, k);
-    if constexpr (TYPE == MXH_Q6_K) {
-        uint8_t* op = o + (size_t)row * row_bytes(MXH_Q6_K, 256 * (int64_t)row_blocks);
-        const Q6KTileOffs f = q6k_tile_offsets(c, row_blocks);
-        const uint8_t* src = rp + (size_t)(c >> 2) * 210;
-        const int h = (c >> 1) & 1, p = c & 1;
-        *reinterpret_cast<uint4*>(op + f.qa) = ld_u16x8(src + 64 * h + 16 * p);
-        *reinterpret_cast<uint4*>(op + f.qb) = ld_u16x8(src + 64 * h + 32 + 16 * p);
-        *reinterpret_cast<uint4*>(op + f.qh) = ld_u16x8(src + 128 + 32 * h + 16 * p);
-        if ((c & 3) == 0) {
-            *reinterpret_cast<uint4*>(op + f.sc) = ld_u16x8(src + 192);
-            *reinterpret_cast<uint16_t*>(op + f.d) = *reinterpret_cast<const uint16_t*>(src + 208);
-        }
-    } else {
-        uint8_t* op = o + (size_t)row * row_bytes(MXH_Q8_0, 256 * (int64_t)row_blocks);
-        const Q80TileOffs f = q80_tile_offsets(c, 8 * row_blocks);
-        uint4 lo, hi;
-        const uint8_t* src;
-        if constexpr (TYPE == MXH_Q8_0) {
-            src = rp + (size_t)c * 34;
-            lo = ld_u16x8(src + 2);
-            hi = ld_u16x8(src + 18);
-        } else {  // Q5_0: d, 32 high bits, 16 bytes of nibbles; code - 16 as a signed byte
-            src = rp + (size_t)c * 22;
-            const uint16_t* h = reinterpret_cast<const uint16_t*>(src);
-            const uint32_t qh = h[1] | ((uint32_t)h[2] << 16);
-            const uint4 qs = ld_u16x8(src + 6);
-            const uint32_t q[4] = {qs.x, qs.y, qs.z, qs.w};
-            uint32_t a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = b[i] = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t byte = (q[i] >> (8 * e)) & 0xffu;
-                    const uint32_t x = (byte & 15u) | (((qh >> (4 * i + e)) & 1u) << 4);
-                    const uint32_t y = (byte >> 4) | (((qh >> (16 + 4 * i + e)) & 1u) << 4);
-                    a[i] |= ((x - 16u) & 0xffu) << (8 * e);
-                    b[i] |= ((y - 16u) & 0xffu) << (8 * e);
-                }
-            }
-            lo = make_uint4(a[0], a[1], a[2], a[3]);
-            hi = make_uint4(b[0], b[1], b[2], b[3]);
-        }
-        *reinterpret_cast<uint4*>(op + f.lo) = lo;
-        *reinterpret_cast<uint4*>(op + f.hi) = hi;
-        *reinterpret_cast<uint16_t*>(op + f.d) = *reinterpret_cast<const uint16_t*>(src);
+    const uint8_t* src = w + (size_t)row * row_bytes(MXH_Q6_K, k) + (size_t)(c >> 2) * 210;
+    uint8_t* op = o + (size_t)row * row_bytes(MXH_Q6_K, 256 * (int64_t)row_blocks);
+    const Q6KTileOffs f = q6k_tile_offsets(c, row_blocks);
+    const int h = (c >> 1) & 1, p = c & 1;
+    *reinterpret_cast<uint4*>(op + f.qa) = ld_u16x8(src + 64 * h + 16 * p);
+    *reinterpret_cast<uint4*>(op + f.qb) = ld_u16x8(src + 64 * h + 32 + 16 * p);
+    *reinterpret_cast<uint4*>(op + f.qh) = ld_u16x8(src + 128 + 32 * h + 16 * p);
+    if ((c & 3) == 0) {
+        *reinterpret_cast<uint4*>(op + f.sc) = ld_u16x8(src + 192);
+        *reinterpret_cast<uint16_t*>(op + f.d) = *reinterpret_cast<const uint16_t*>(src + 208);
     }
 }
 
@@ -898,23 +949,28 @@ struct Plan {
 };
 
 // The tile shape and split of K with the lowest estimate of
-//   rounds of the 256 CUs x (steps of a work item x time of a step + 7.5 us)
+//   rounds of the 256 CUs x (steps of a work item x time of a step + its start)
 //   + the reduction of the partial tiles,
 // the step's time lying between what it takes on a nearly idle chip and on a
 // full one (ns, measured per format and tile at K = 4096 .. 14336, where the
 // estimate is within 10% of the measured time of the shapes tried); 7.5 us is
-// what a work item takes to start, fill its stages and store its outputs.
+// what a work item takes to start, fill its stages and store its outputs.  The
+// rows in GGUF order were fitted from K = 1024 on, with that time per tile too
+// (rms 5 to 9%).
 Plan gemm_plan(int fmt, int m, int n, int k) {
     struct Cost {
-        float idle, full;
+        float idle, full, item = 7500.f;
     };
-    static const Cost cost[4][GT_COUNT] = {
+    static const Cost cost[6][GT_COUNT] = {
         {{1420.f, 2130.f}, {830.f, 1160.f}, {800.f, 1110.f}, {490.f, 650.f}},       // Q4_K
         {{1680.f, 2280.f}, {980.f, 1270.f}, {950.f, 1220.f}, {650.f, 830.f}},       // Q5_K
         {{1720.f, 2300.f}, {980.f, 1180.f}, {950.f, 1200.f}, {600.f, 830.f}},       // Q8_0
-        {{1e6f, 1e6f}, {1430.f, 1730.f}, {1560.f, 1830.f}, {1000.f, 1130.f}}};      // Q6_K
+        {{1e6f, 1e6f}, {1430.f, 1730.f}, {1560.f, 1830.f}, {1000.f, 1130.f}},       // Q6_K
+        {{1880.f, 2180.f, 8000.f}, {960.f, 1210.f, 4300.f}, {1070.f, 1280.f, 4400.f}, {830.f, 990.f, 2500.f}},  // Q8_0 in GGUF order
+        {{2460.f, 2470.f, 9100.f}, {1350.f, 1350.f, 5300.f}, {1250.f, 1280.f, 5500.f}, {1140.f, 780.f, 2000.f}}};  // Q5_0
     static const int bm[GT_COUNT] = {128, 128, 64, 32}, bn[GT_COUNT] = {256, 128, 256, 256};
-    const int cls = fmt == GF_Q80T ? 2 : fmt == GF_Q6KT ? 3 : fmt == GF_Q5K || fmt == GF_Q5KT ? 1 : 0, nblk = k / 256;
+    static const int cls_of[] = {0, 0, 1, 1, 4, 2, 5, 3};  // by GemmFmt
+    const int cls = cls_of[fmt], nblk = k / 256;
     Plan best{GT_128x256, nblk, 1};
     double best_cost = 1e30;
     for (int t = cls == 3 ? GT_128x128 : GT_128x256; t < GT_COUNT; ++t) {
@@ -924,10 +980,10 @@ Plan gemm_plan(int fmt, int m, int n, int k) {
             if ((nblk + blocks - 1) / blocks != s) continue;
             const double floats = (double)s * m * n;
             if (s > 1 && floats * 4 > (double)kPartBytes) break;
+            const Cost& c = cost[cls][t];
             const int64_t items = tiles * s, rounds = (items + 255) / 256;
             const double load = items >= 256 ? 1.0 : items / 256.0;
-            const Cost& c = cost[cls][t];
-            const double ns = rounds * (4.0 * blocks * (c.idle + load * (c.full - c.idle)) + 7500.0) +
+            const double ns = rounds * (4.0 * blocks * (c.idle + load * (c.full - c.idle)) + c.item) +
                               (s > 1 ? 3000.0 + floats * 4 / 3000.0 : 0.0);
             if (ns < best_cost) {
                 best_cost = ns;
@@ -983,19 +1039,20 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
     case MXH_Q4_K_TILED: f = GF_Q4KT; break;
     case MXH_Q5_K: f = GF_Q5K; break;
     case MXH_Q5_K_TILED: f = GF_Q5KT; break;
+    case MXH_Q8_0: f = GF_Q80; break;
     case MXH_Q8_0_TILED: f = GF_Q80T; break;
+    case MXH_Q5_0: f = GF_Q50; break;
     case MXH_Q6_K_TILED: f = GF_Q6KT; break;
-    case MXH_Q6_K:
+    default:  // Q6_K
         f = GF_Q6KT, regroup = true;
         a.row_blocks = (a.row_blocks + 7) / 8 * 8;
         break;
-    default: f = GF_Q80T, regroup = true; break;
     }
     if (!regroup && !al16(w)) return MXH_ERR_ARG;
     const Plan p = gemm_plan(f, m, n, k);
     a.blocks = p.blocks, a.splits = p.splits;
     const size_t in_rb = row_bytes(type, k);
-    const size_t rb = regroup ? row_bytes(f == GF_Q6KT ? MXH_Q6_K : MXH_Q8_0, 256 * (int64_t)a.row_blocks) : in_rb;
+    const size_t rb = row_bytes(MXH_Q6_K, 256 * (int64_t)a.row_blocks);  // of a regrouped row
     // regrouped rows go through the slab, whole tiles of rows at a time
     const int step = regroup ? (int)std::min<size_t>((size_t)n, kSlabBytes / rb / 256 * 256) : n;
     for (int n0 = 0; n0 < n; n0 += step) {
@@ -1003,14 +1060,9 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
         const uint8_t* src = static_cast<const uint8_t*>(w) + (size_t)n0 * in_rb;
         a.w = src;
         if (regroup) {
-            const int64_t threads = (int64_t)nn * (k / (type == MXH_Q6_K ? 64 : 32));
-            const dim3 grid((unsigned)((threads + 255) / 256));
-            if (type == MXH_Q8_0)
-                hipLaunchKernelGGL(regroup_rows_kernel<MXH_Q8_0>, grid, dim3(256), 0, st, src, g_slab_ptr, nn, k, a.row_blocks);
-            else if (type == MXH_Q5_0)
-                hipLaunchKernelGGL(regroup_rows_kernel<MXH_Q5_0>, grid, dim3(256), 0, st, src, g_slab_ptr, nn, k, a.row_blocks);
-            else
-                hipLaunchKernelGGL(regroup_rows_kernel<MXH_Q6_K>, grid, dim3(256), 0, st, src, g_slab_ptr, nn, k, a.row_blocks);
+            const int64_t threads = (int64_t)nn * (k / 64);
+            hipLaunchKernelGGL(regroup_q6k_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, src,
+                               g_slab_ptr, nn, k, a.row_blocks);
             a.w = g_slab_ptr;
         }
         a.n = nn;

@@ -8,7 +8,7 @@
 namespace mxh {
 
 // weight formats (GGUF block order, T: the tiled order of mxh_types.h)
-enum GemmFmt { GF_Q4K, GF_Q4KT, GF_Q5K, GF_Q5KT, GF_Q80T, GF_Q6KT };
+enum GemmFmt { GF_Q4K, GF_Q4KT, GF_Q5K, GF_Q5KT, GF_Q80, GF_Q80T, GF_Q50, GF_Q6KT };
 
 // out[m x n] (row stride ldo) = a . W^T (+ res), a as fp16 hi / lo of a 2^e
 // per row (row stride lda), s: split sums of every 32-element sub-block (row
