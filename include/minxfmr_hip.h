@@ -151,12 +151,15 @@ int mxh_gemm_q_bf16(int type, const float *a, int64_t m, const void *w, int64_t 
  * Q5_K, Q8_0 or Q5_0 (or a tiled id of mxh_tile_rows), k a multiple of 256 up
  * to 16384.  The prefill contraction the model runs: the reference's
  * backend_matmul_rhs_transposed with m > 1
- * (src/backend/backend_runtime.cpp:302-319). */
+ * (src/backend/backend_runtime.cpp:302-319).  Partial sums of split K go
+ * through 64 MiB of static device memory that every launch on the library
+ * stream shares, in stream order. */
 int mxh_gemm_q_f16(int type, const float *a, int64_t m, const void *w, int64_t n, int64_t k, float *out, int form);
 
 /* mxh_gemm_q_f16 without any allocation: the staged activations live in a
- * device scratch array of 12 MiB that every GPU the library runs on holds
- * from load until the process ends, so 4 m k + m k / 8 + 4 m bytes (about
+ * device scratch array of 12 MiB, partial sums in another of 64 MiB, that
+ * every GPU the library runs on holds from load until the process ends and no
+ * other entry uses (but mxh_gemm_q_f16 recorded in a graph), so 4 m k + m k / 8 + 4 m bytes (about
  * 4.1 bytes per element of a) must fit in it; larger requests are rejected
  * with MXH_ERR_ARG and a message.  Calls no hipMalloc / hipFree; results are
  * identical to mxh_gemm_q_f16's.  Every call on a GPU reuses that GPU's
@@ -173,7 +176,11 @@ int mxh_gemm_q_f16_noalloc(int type, const float *a, int64_t m, const void *w, i
  * cores; device pointers.  q: [m][nh*hd] fp32 (after RoPE); kc, vc: the fp16
  * cache [>= p0+m][nkv*hd] with rows 0 .. p0+m-1 written; att: [m][nh*hd].
  * nh a multiple of nkv with at most 8 q heads per kv head, hd 32, 64 or 128.
- * The batched prefill's attention step. */
+ * The batched prefill's attention step.  Few queries over many keys split the
+ * keys among workgroups, their parts going through the library stream's shared
+ * static memory (see mxh_gemm_q_f16); recorded in a graph (the library stream
+ * capturing) a call does not split, so its replays use the caller's buffers
+ * alone and may overlap anything. */
 int mxh_attention_prefill(const float *q, const void *kc, const void *vc, float *att, int p0, int m, int nh, int nkv,
                           int hd);
 

@@ -72,15 +72,22 @@ int ensure_ready() {
     return mxh_init(0);
 }
 
+// whether launches are being recorded in a caller's graph: its replays may run
+// beside the library stream, so they keep off what launches there share
+bool capturing() {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(g_ctx.stream, &s) == hipSuccess && s == hipStreamCaptureStatusActive;
+}
+
 // validation and the two launches of mxh_gemm_q_f16 over staging at `buf`
 int gemm_q_f16_body(const char* who, int type, const float* a, int64_t m, const void* w, int64_t n, int64_t k,
-                    float* out, int form, void* buf) {
+                    float* out, int form, void* buf, Workspace ws) {
     const F16Rows r = f16_rows_layout(buf, (size_t)m, (size_t)k);
     if (int rc = rows_to_f16_launch(a, (int)k, nullptr, 0.f, (int)k, r.a_hi, r.a_lo, (int)k, r.s_hi, r.s_lo,
                                     (int)k / 32, r.rscale, (int)m, g_ctx.stream))
         return set_error(rc, "%s: conversion launch", who);
     if (int rc = gemm_q_f16_run(type, r.a_hi, r.a_lo, (int)k, r.s_hi, r.s_lo, (int)k / 32, r.rscale, w, out, (int)n,
-                                nullptr, (int)m, (int)n, (int)k, form, g_ctx.stream))
+                                nullptr, (int)m, (int)n, (int)k, form, ws, g_ctx.stream))
         return set_error(rc, "%s: launch", who);
     return check_hip(hipGetLastError(), who);
 }
@@ -350,7 +357,8 @@ int mxh_gemm_q_f16(int type, const float* a, int64_t m, const void* w, int64_t n
     if (int rc = gemm_q_f16_check("gemm_f16", type, a, m, w, n, k, out)) return rc;
     void* buf = nullptr;
     if (int rc = stage(2, f16_rows_bytes((size_t)m, (size_t)k), &buf)) return rc;
-    return gemm_q_f16_body("gemm_f16", type, a, m, w, n, k, out, form, buf);
+    return gemm_q_f16_body("gemm_f16", type, a, m, w, n, k, out, form, buf,
+                           capturing() ? Workspace::kNoalloc : Workspace::kStream);
 }
 
 int mxh_gemm_q_f16_noalloc(int type, const float* a, int64_t m, const void* w, int64_t n, int64_t k, float* out,
@@ -363,7 +371,7 @@ int mxh_gemm_q_f16_noalloc(int type, const float* a, int64_t m, const void* w, i
                          kNoallocScratchBytes);
     void* buf = g_scratch_ptr[g_ctx.device];
     if (!buf) return set_error(MXH_ERR_HIP, "gemm_f16_noalloc: no scratch address for device %d", g_ctx.device);
-    return gemm_q_f16_body("gemm_f16_noalloc", type, a, m, w, n, k, out, form, buf);
+    return gemm_q_f16_body("gemm_f16_noalloc", type, a, m, w, n, k, out, form, buf, Workspace::kNoalloc);
 }
 
 int mxh_attention_prefill(const float* q, const void* kc, const void* vc, float* att, int p0, int m, int nh, int nkv,
@@ -373,8 +381,10 @@ int mxh_attention_prefill(const float* q, const void* kc, const void* vc, float*
     if (m <= 0 || p0 < 0 || !attention_supported(nh, nkv, hd))
         return set_error(MXH_ERR_ARG, "attention_prefill: unsupported m %d p0 %d nh %d nkv %d hd %d", m, p0, nh, nkv,
                          hd);
+    size_t part_bytes = 0;
+    float* part = capturing() ? nullptr : reinterpret_cast<float*>(gemm_partials(&part_bytes));
     if (int rc = attention_rows_mfma_launch(q, (const __half*)kc, (const __half*)vc, att, p0, m, nh, nkv, hd,
-                                            1.0f / sqrtf((float)hd), g_ctx.stream))
+                                            1.0f / sqrtf((float)hd), part, part_bytes, g_ctx.stream))
         return set_error(rc, "attention_prefill: launch");
     return check_hip(hipGetLastError(), "attention_prefill launch");
 }

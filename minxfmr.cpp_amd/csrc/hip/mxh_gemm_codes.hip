@@ -906,12 +906,12 @@ void reduce_launch(const float* part, int splits, float* out, int ldo, const flo
 
 // Device workspace of the GEMMs, held by every GPU the library runs on from
 // load until the process ends, so that no call allocates: partial tiles of
-// split K, and a slab of rows regrouped for the kernel.  Every launch that
-// uses it is on the library stream.
+// split K (one array per Workspace), and a slab of rows regrouped for the
+// kernel.
 constexpr size_t kPartBytes = 64u << 20, kSlabBytes = 64u << 20;
-static __device__ __align__(256) uint8_t g_partials[kPartBytes];
+static __device__ __align__(256) uint8_t g_partials[2][kPartBytes];
 static __device__ __align__(256) uint8_t g_slab[kSlabBytes];
-float* g_part_ptr = nullptr;
+float* g_part_ptr[2] = {nullptr, nullptr};
 uint8_t* g_slab_ptr = nullptr;
 
 // Q6_K rows in GGUF order are only 2-aligned (210-byte blocks): regrouped into
@@ -1000,14 +1000,14 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 uint8_t* gemm_partials(size_t* bytes) {
     *bytes = kPartBytes;
-    return reinterpret_cast<uint8_t*>(g_part_ptr);
+    return reinterpret_cast<uint8_t*>(g_part_ptr[(int)Workspace::kStream]);
 }
 
 int gemm_workspace_init() {
     void *p = nullptr, *q = nullptr;
     if (int rc = check_hip(hipGetSymbolAddress(&p, HIP_SYMBOL(g_partials)), "hipGetSymbolAddress(partials)")) return rc;
     if (int rc = check_hip(hipGetSymbolAddress(&q, HIP_SYMBOL(g_slab)), "hipGetSymbolAddress(slab)")) return rc;
-    g_part_ptr = static_cast<float*>(p);
+    for (int i = 0; i < 2; ++i) g_part_ptr[i] = reinterpret_cast<float*>(static_cast<uint8_t*>(p) + i * kPartBytes);
     g_slab_ptr = static_cast<uint8_t*>(q);
     return MXH_OK;
 }
@@ -1024,13 +1024,14 @@ bool gemm_q_f16_supported(int type, int k) {
 
 int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda, const uint16_t* s_hi,
                    const uint16_t* s_lo, int lds, const float* rscale, const void* w, float* out, int ldo,
-                   const float* res, int m, int n, int k, int form, hipStream_t st) {
+                   const float* res, int m, int n, int k, int form, Workspace ws, hipStream_t st) {
     if (m <= 0 || n <= 0 || !gemm_q_f16_supported(type, k) || lda < k || lds < k / 32 || ldo < n) return MXH_ERR_ARG;
+    float* part = g_part_ptr[(int)ws];
     // the direct loads are 16 bytes wide
-    if (!al16(a_hi) || !al16(a_lo) || !al16(s_hi) || !al16(s_lo) || lda % 8 || lds % 8 || !g_part_ptr) return MXH_ERR_ARG;
+    if (!al16(a_hi) || !al16(a_lo) || !al16(s_hi) || !al16(s_lo) || lda % 8 || lds % 8 || !part) return MXH_ERR_ARG;
     CodesArgs a{};
     a.a_hi = a_hi, a.a_lo = a_lo, a.s_hi = s_hi, a.s_lo = s_lo, a.rscale = rscale;
-    a.out = out, a.res = res, a.part = g_part_ptr;
+    a.out = out, a.res = res, a.part = part;
     a.lda = lda, a.lds = lds, a.ldo = ldo, a.m = m, a.n = n, a.k = k, a.form = form, a.row_blocks = k / 256;
     GemmFmt f;
     bool regroup = false;
@@ -1048,7 +1049,7 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
         a.row_blocks = (a.row_blocks + 7) / 8 * 8;
         break;
     }
-    if (!regroup && !al16(w)) return MXH_ERR_ARG;
+    if (regroup ? ws != Workspace::kStream : !al16(w)) return MXH_ERR_ARG;  // (one slab)
     const Plan p = gemm_plan(f, m, n, k);
     a.blocks = p.blocks, a.splits = p.splits;
     const size_t in_rb = row_bytes(type, k);

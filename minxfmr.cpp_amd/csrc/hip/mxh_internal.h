@@ -123,15 +123,18 @@ int gemm_bf16_run(int type, const uint16_t* a, const uint16_t* a_lo, int lda, co
 // multiple of 256 up to 16384.  a as fp16 hi / lo of a * 2^e per row, s the
 // split sums of every 32-element sub-block of those values (row stride lds),
 // rscale = 2^-e per row; inputs from rows_to_f16 / silu_mul_f16.  Its
-// workspace is static device memory (gemm_workspace_init, once per process):
-// calls run on the library stream.
+// workspace is static device memory (gemm_workspace_init, once per process) in
+// two parts that share nothing: kStream for launches that run on the library
+// stream, one after the other; kNoalloc for mxh_gemm_q_f16_noalloc and for
+// launches recorded in a caller's graph, which may run beside that stream.
+enum class Workspace { kStream, kNoalloc };
 int gemm_workspace_init();
-// its part for partial sums, which other kernels on the library stream may use between GEMMs
+// kStream's partial sums, which other launches that run on the library stream may use between GEMMs
 uint8_t* gemm_partials(size_t* bytes);
 bool gemm_q_f16_supported(int type, int k);
 int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda, const uint16_t* s_hi,
                    const uint16_t* s_lo, int lds, const float* rscale, const void* w, float* out, int ldo,
-                   const float* res, int m, int n, int k, int form, hipStream_t st);
+                   const float* res, int m, int n, int k, int form, Workspace ws, hipStream_t st);
 int rows_to_f16_launch(const float* x, int ldx, const float* nw, float eps, int k, uint16_t* a_hi, uint16_t* a_lo,
                        int lda, uint16_t* s_hi, uint16_t* s_lo, int lds, float* rscale, int m, hipStream_t st);
 int silu_mul_f16_launch(const float* gu, int f, uint16_t* h_hi, uint16_t* h_lo, uint16_t* s_hi, uint16_t* s_lo,
@@ -171,9 +174,10 @@ int qkv_prep_rows_launch(const float* qkv, int ldq, const float* bias, const flo
                          const double* rope_cs, int p0, int m, float* q_out, __half* kc, __half* vc, int nh, int nkv,
                          int hd, int neox, float eps, hipStream_t st);
 // causal attention of prompt tokens p0 .. p0+m-1 over the fp16 cache, on the
-// fp16 matrix cores (mxh_prefill_attn.hip)
+// fp16 matrix cores (mxh_prefill_attn.hip); `part` (part_bytes of scratch, may
+// be null) lets few queries split their keys among workgroups
 int attention_rows_mfma_launch(const float* q, const __half* kc, const __half* vc, float* att, int p0, int m, int nh,
-                               int nkv, int hd, float scale, hipStream_t st);
+                               int nkv, int hd, float scale, float* part, size_t part_bytes, hipStream_t st);
 int embed_rows_launch(int type, const void* w, const int* tokens, int p0, int m, float* x, int cols, int form,
                       hipStream_t st);
 

@@ -778,7 +778,7 @@ bool f16_gemm(const mxh_model* m, const DevW& w) {
 int gemm(mxh_model* m, const DevW& w, int lda, float* out, int ldo, const float* res, int rows, hipStream_t st) {
     if (f16_gemm(m, w))
         return gemm_q_f16_run(w.type, m->pf_h16, m->pf_l16, lda, m->pf_sh, m->pf_sl, lda / 32, m->pf_rscale, w.p,
-                                out, ldo, res, rows, (int)w.rows, (int)w.cols, m->form, st);
+                                out, ldo, res, rows, (int)w.rows, (int)w.cols, m->form, Workspace::kStream, st);
     return gemm_bf16_run(w.type, m->pf_a, m->pf_a_lo, lda, w.p, out, ldo, res, rows, (int)w.rows, (int)w.cols,
                          m->form, m->pf_part, m->pf_part_floats, st);
 }
@@ -806,6 +806,8 @@ int enqueue_prefill_chunk(mxh_model* m, int p0, int rows, hipStream_t st) {
     const mxh_model_config& c = m->cfg;
     const int d = c.n_embd, hd = c.head_dim, nh = c.n_head, nkv = c.n_head_kv, f = c.n_ff;
     const int qd = nh * hd, kvd = nkv * hd, ldq = qd + 2 * kvd;
+    size_t part_bytes = 0;  // the attention's key splits, between the GEMMs
+    float* part = reinterpret_cast<float*>(gemm_partials(&part_bytes));
     int rc = embed_rows_launch(m->embd.type, m->embd.p, m->tokens, p0, rows, m->pf_x, d, m->form, st);
     for (int l = 0; l < c.n_layer && !rc; ++l) {
         const Layer& L = m->layers[(size_t)l];
@@ -820,7 +822,7 @@ int enqueue_prefill_chunk(mxh_model* m, int p0, int rows, hipStream_t st) {
         rc |= qkv_prep_rows_launch(m->pf_qkv, ldq, L.bias, L.q_norm, L.k_norm, m->rope_cs, p0, rows, m->pf_q, L.kc,
                                    L.vc, nh, nkv, hd, m->neox, c.eps, st);
         rc |= attention_rows_mfma_launch(m->pf_q, L.kc, L.vc, m->pf_att, p0, rows, nh, nkv, hd, 1.0f / sqrtf((float)hd),
-                                          st);
+                                         part, part_bytes, st);
         rc |= prep_rows(m, {&L.o}, m->pf_att, qd, nullptr, 0.f, qd, rows, st);
         rc |= gemm(m, L.o, qd, m->pf_x, d, m->pf_x, rows, st);
         rc |= prep_rows(m, {&L.gu, &L.g, &L.u}, m->pf_x, d, L.ffn_norm, c.eps, d, rows, st);

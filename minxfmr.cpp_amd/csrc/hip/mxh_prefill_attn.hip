@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(const float* 
 constexpr int kPaSplitsMax = 32;
 template <int HD>
 int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half* vc, float* att, int p0, int m,
-                                  int nh, int nkv, float qscale, hipStream_t st) {
+                                  int nh, int nkv, float qscale, float* part, size_t part_bytes, hipStream_t st) {
     static bool attr_set = false;  // above 64 KiB of LDS needs the opt-in, once per kernel
     if (!attr_set) {
         if (hipFuncSetAttribute((const void*)attention_rows_mfma_kernel<HD>,
@@ -408,13 +408,11 @@ int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half
     const int T = kPaRows / (nh / nkv), tiles = (m + T - 1) / T;
     const int64_t wgs = (int64_t)nkv * tiles;
     const int stages = (int)(((int64_t)p0 + m + kPaKeys - 1) / kPaKeys);
-    size_t part_bytes = 0;
-    float* part = reinterpret_cast<float*>(gemm_partials(&part_bytes));
     int splits = 1, per = stages;
     double best = 1e30;
     for (int s = 1; s <= kPaSplitsMax && s <= stages; ++s) {
         const size_t bytes = (size_t)wgs * s * kPaRows * (HD + 2) * 4;
-        if (s > 1 && bytes > part_bytes) break;
+        if (s > 1 && (!part || bytes > part_bytes)) break;
         const int p = (stages + s - 1) / s;
         if ((stages + p - 1) / p != s) continue;  // the same stages in fewer splits
         const int64_t on_cu = (wgs * s + kCus - 1) / kCus, rounds = (on_cu + kSlots - 1) / kSlots;
@@ -423,7 +421,8 @@ int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half
         if (s > 1) us += 3.5 + 0.3 * s + (double)bytes / 5e6;
         if (us < best) best = us, splits = s, per = p;
     }
-    float2* ml = reinterpret_cast<float2*>(part + (size_t)wgs * splits * kPaRows * HD);  // (splits > 1)
+    // (used with splits > 1 only)
+    float2* ml = part ? reinterpret_cast<float2*>(part + (size_t)wgs * splits * kPaRows * HD) : nullptr;
     hipLaunchKernelGGL(attention_rows_mfma_kernel<HD>, dim3((unsigned)nkv, (unsigned)tiles, (unsigned)splits),
                        dim3(kPaThreads), pa_lds_bytes(HD), st, q, kc, vc, att, part, ml, p0, m, nh, nkv, qscale, per);
     if (splits > 1) {
@@ -437,13 +436,13 @@ int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half
 }  // namespace
 
 int attention_rows_mfma_launch(const float* q, const __half* kc, const __half* vc, float* att, int p0, int m, int nh,
-                               int nkv, int hd, float scale, hipStream_t st) {
+                               int nkv, int hd, float scale, float* part, size_t part_bytes, hipStream_t st) {
     if (m <= 0 || p0 < 0 || !attention_supported(nh, nkv, hd)) return MXH_ERR_ARG;
     const float qscale = scale * 1.4426950408889634f;  // scores in base-2 units
     switch (hd) {
-    case 32: return attention_rows_mfma_launch_hd<32>(q, kc, vc, att, p0, m, nh, nkv, qscale, st);
-    case 64: return attention_rows_mfma_launch_hd<64>(q, kc, vc, att, p0, m, nh, nkv, qscale, st);
-    default: return attention_rows_mfma_launch_hd<128>(q, kc, vc, att, p0, m, nh, nkv, qscale, st);
+    case 32: return attention_rows_mfma_launch_hd<32>(q, kc, vc, att, p0, m, nh, nkv, qscale, part, part_bytes, st);
+    case 64: return attention_rows_mfma_launch_hd<64>(q, kc, vc, att, p0, m, nh, nkv, qscale, part, part_bytes, st);
+    default: return attention_rows_mfma_launch_hd<128>(q, kc, vc, att, p0, m, nh, nkv, qscale, part, part_bytes, st);
     }
 }
 
