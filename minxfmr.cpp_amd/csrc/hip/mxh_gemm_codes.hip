@@ -1050,12 +1050,14 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
         break;
     }
     if (regroup ? ws != Workspace::kStream : !al16(w)) return MXH_ERR_ARG;  // (one slab)
-    const Plan p = gemm_plan(f, m, n, k);
-    a.blocks = p.blocks, a.splits = p.splits;
     const size_t in_rb = row_bytes(type, k);
     const size_t rb = row_bytes(MXH_Q6_K, 256 * (int64_t)a.row_blocks);  // of a regrouped row
-    // regrouped rows go through the slab, whole tiles of rows at a time
-    const int step = regroup ? (int)std::min<size_t>((size_t)n, kSlabBytes / rb / 256 * 256) : n;
+    // regrouped rows go through the slab in equal pieces, whole tiles of rows,
+    // each under the plan for what it launches (2 x 30000 x 11008 under a plan
+    // for all rows: seven launches of a seventh of the chip)
+    const int slab_rows = regroup ? (int)(kSlabBytes / rb / 256 * 256) : n;
+    const int pieces = (n - 1) / slab_rows + 1;
+    const int step = pieces > 1 ? ((n - 1) / pieces + 256) / 256 * 256 : n;
     for (int n0 = 0; n0 < n; n0 += step) {
         const int nn = std::min(step, n - n0);
         const uint8_t* src = static_cast<const uint8_t*>(w) + (size_t)n0 * in_rb;
@@ -1066,6 +1068,8 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
                                g_slab_ptr, nn, k, a.row_blocks);
             a.w = g_slab_ptr;
         }
+        const Plan p = gemm_plan(f, m, nn, k);
+        a.blocks = p.blocks, a.splits = p.splits;
         a.n = nn;
         a.out = out + n0;
         a.res = res ? res + n0 : nullptr;
