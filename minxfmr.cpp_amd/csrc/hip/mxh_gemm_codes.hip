@@ -943,57 +943,6 @@ __global__ __launch_bounds__(256) void regroup_q6k_kernel(const uint8_t* __restr
     }
 }
 
-struct Plan {
-    GemmTile tile;
-    int blocks, splits;
-};
-
-// The tile shape and split of K with the lowest estimate of
-//   rounds of the 256 CUs x (steps of a work item x time of a step + its start)
-//   + the reduction of the partial tiles,
-// the step's time lying between what it takes on a nearly idle chip and on a
-// full one (ns, measured per format and tile at K = 4096 .. 14336, where the
-// estimate is within 10% of the measured time of the shapes tried); 7.5 us is
-// what a work item takes to start, fill its stages and store its outputs.  The
-// rows in GGUF order were fitted from K = 1024 on, with that time per tile too
-// (rms 5 to 9%).
-Plan gemm_plan(int fmt, int m, int n, int k) {
-    struct Cost {
-        float idle, full, item = 7500.f;
-    };
-    static const Cost cost[6][GT_COUNT] = {
-        {{1420.f, 2130.f}, {830.f, 1160.f}, {800.f, 1110.f}, {490.f, 650.f}},       // Q4_K
-        {{1680.f, 2280.f}, {980.f, 1270.f}, {950.f, 1220.f}, {650.f, 830.f}},       // Q5_K
-        {{1720.f, 2300.f}, {980.f, 1180.f}, {950.f, 1200.f}, {600.f, 830.f}},       // Q8_0
-        {{1e6f, 1e6f}, {1430.f, 1730.f}, {1560.f, 1830.f}, {1000.f, 1130.f}},       // Q6_K
-        {{1880.f, 2180.f, 8000.f}, {960.f, 1210.f, 4300.f}, {1070.f, 1280.f, 4400.f}, {830.f, 990.f, 2500.f}},  // Q8_0 in GGUF order
-        {{2460.f, 2470.f, 9100.f}, {1350.f, 1350.f, 5300.f}, {1250.f, 1280.f, 5500.f}, {1140.f, 780.f, 2000.f}}};  // Q5_0
-    static const int bm[GT_COUNT] = {128, 128, 64, 32}, bn[GT_COUNT] = {256, 128, 256, 256};
-    static const int cls_of[] = {0, 0, 1, 1, 4, 2, 5, 3};  // by GemmFmt
-    const int cls = cls_of[fmt], nblk = k / 256;
-    Plan best{GT_128x256, nblk, 1};
-    double best_cost = 1e30;
-    for (int t = cls == 3 ? GT_128x128 : GT_128x256; t < GT_COUNT; ++t) {
-        const int64_t tiles = (int64_t)((n + bn[t] - 1) / bn[t]) * ((m + bm[t] - 1) / bm[t]);
-        for (int s = 1; s <= nblk && s <= 32; ++s) {
-            const int blocks = (nblk + s - 1) / s;
-            if ((nblk + blocks - 1) / blocks != s) continue;
-            const double floats = (double)s * m * n;
-            if (s > 1 && floats * 4 > (double)kPartBytes) break;
-            const Cost& c = cost[cls][t];
-            const int64_t items = tiles * s, rounds = (items + 255) / 256;
-            const double load = items >= 256 ? 1.0 : items / 256.0;
-            const double ns = rounds * (4.0 * blocks * (c.idle + load * (c.full - c.idle)) + c.item) +
-                              (s > 1 ? 3000.0 + floats * 4 / 3000.0 : 0.0);
-            if (ns < best_cost) {
-                best_cost = ns;
-                best = Plan{(GemmTile)t, blocks, s};
-            }
-        }
-    }
-    return best;
-}
-
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -1068,7 +1017,7 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
                                g_slab_ptr, nn, k, a.row_blocks);
             a.w = g_slab_ptr;
         }
-        const Plan p = gemm_plan(f, m, nn, k);
+        const GemmPlan p = gemm_plan(f, m, nn, k, device_cus(), kPartBytes);
         a.blocks = p.blocks, a.splits = p.splits;
         a.n = nn;
         a.out = out + n0;

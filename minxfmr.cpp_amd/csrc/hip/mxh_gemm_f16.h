@@ -5,10 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace mxh {
+#include "mxh_plan.h"
 
-// weight formats (GGUF block order, T: the tiled order of mxh_types.h)
-enum GemmFmt { GF_Q4K, GF_Q4KT, GF_Q5K, GF_Q5KT, GF_Q80, GF_Q80T, GF_Q50, GF_Q6KT };
+namespace mxh {
 
 // out[m x n] (row stride ldo) = a . W^T (+ res), a as fp16 hi / lo of a 2^e
 // per row (row stride lda), s: split sums of every 32-element sub-block (row
@@ -26,8 +25,6 @@ struct CodesArgs {
     int lda, lds, ldo, m, n, k, form, row_blocks, blocks, splits;
 };
 
-// tile shapes of the kernel (activation rows x weight rows)
-enum GemmTile { GT_128x256, GT_128x128, GT_64x256, GT_32x256, GT_COUNT };
 int gemm_codes_launch(GemmFmt f, GemmTile t, const CodesArgs& a, hipStream_t st);
 
 }  // namespace mxh

@@ -1434,16 +1434,6 @@ __global__ __launch_bounds__(1024) void argmax_finish_kernel(const float* __rest
 // Resident workgroups of a kernel on the whole device (occupancy x CUs),
 // cached per kernel and LDS size: a persistent grid of exactly this size runs
 // in one round, so each resident slot stages x once.
-int device_cus() {
-    static int n_cu = 0;
-    if (!n_cu) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            n_cu = 256;
-    }
-    return n_cu;
-}
-
 int resident_grid(const void* kernel, size_t lds, int threads) {
     struct Entry {
         const void* k;
@@ -1672,6 +1662,16 @@ int rows_launch(const uint8_t* w, const float* x, float* y, int m, int n, int k,
 }
 
 }  // namespace
+
+int device_cus() {
+    static int n_cu = 0;
+    if (!n_cu) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n_cu = 256;
+    }
+    return n_cu;
+}
 
 // max K whose padded x fits the 64 KiB of LDS one workgroup may use
 constexpr int64_t kGemvMaxK = 15360;

@@ -15,6 +15,8 @@ int set_error(int code, const char* fmt, ...);
 int check_hip(hipError_t e, const char* what);
 
 hipStream_t lib_stream();
+// compute units of the current device
+int device_cus();
 
 int gemv_launch(int type, const void* w, const float* x, float* y, const float* res, int64_t n, int64_t k, int form,
                 hipStream_t st);

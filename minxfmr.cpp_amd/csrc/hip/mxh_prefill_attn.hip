@@ -54,6 +54,7 @@
 
 #include "mxh_device.h"
 #include "mxh_internal.h"
+#include "mxh_plan.h"
 
 namespace mxh {
 
@@ -383,15 +384,6 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(const float* 
         make_float4(s.x * inv, s.y * inv, s.z * inv, s.w * inv);
 }
 
-// Splits of the keys among workgroups.  Measured: a stage takes kStage us
-// alone (latencies) and at least kFull us of a CU's time for each workgroup on
-// it, and kSlots workgroups fit a CU; a merge costs its launch (3.5 us), a
-// little a split, and the parts' way through memory.  us without splits / with
-// the splits chosen (m at p0, q heads / kv heads x head dim):
-//   16 at 7680, 32/8 x 128   146 / 22      2 at 7000, 8/1 x 64     90 / 13
-//   128 at 4000, 32/8 x 128   85 / 37      100 at 3000, 8/1 x 32   36 / 12
-//   512 at 7680, 32/8 x 128  210 / 183     512 at 7680, 16/8 x 64 115 / 56
-constexpr int kPaSplitsMax = 32;
 template <int HD>
 int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half* vc, float* att, int p0, int m,
                                   int nh, int nkv, float qscale, float* part, size_t part_bytes, hipStream_t st) {
@@ -402,25 +394,11 @@ int attention_rows_mfma_launch_hd(const float* q, const __half* kc, const __half
             return MXH_ERR_HIP;
         attr_set = true;
     }
-    constexpr double kStart = 4.0, kStage = HD == 128 ? 1.45 : HD == 64 ? 0.85 : 0.7;
-    constexpr double kFull = HD == 128 ? 1.3 : HD == 64 ? 0.75 : 0.5;
-    constexpr int kCus = 256, kSlots = HD == 128 ? 2 : HD == 64 ? 3 : 4;
     const int T = kPaRows / (nh / nkv), tiles = (m + T - 1) / T;
     const int64_t wgs = (int64_t)nkv * tiles;
-    const int stages = (int)(((int64_t)p0 + m + kPaKeys - 1) / kPaKeys);
-    int splits = 1, per = stages;
-    double best = 1e30;
-    for (int s = 1; s <= kPaSplitsMax && s <= stages; ++s) {
-        const size_t bytes = (size_t)wgs * s * kPaRows * (HD + 2) * 4;
-        if (s > 1 && (!part || bytes > part_bytes)) break;
-        const int p = (stages + s - 1) / s;
-        if ((stages + p - 1) / p != s) continue;  // the same stages in fewer splits
-        const int64_t on_cu = (wgs * s + kCus - 1) / kCus, rounds = (on_cu + kSlots - 1) / kSlots;
-        const double full = kFull * (double)on_cu, alone = kStage * (double)rounds;
-        double us = kStart * (double)rounds + p * (full > alone ? full : alone);
-        if (s > 1) us += 3.5 + 0.3 * s + (double)bytes / 5e6;
-        if (us < best) best = us, splits = s, per = p;
-    }
+    const AttnPlan plan = attention_plan(HD, wgs, (int)(((int64_t)p0 + m + kPaKeys - 1) / kPaKeys),
+                                         (size_t)kPaRows * (HD + 2) * 4, device_cus(), part ? part_bytes : 0);
+    const int splits = plan.splits, per = plan.stages;
     // (used with splits > 1 only)
     float2* ml = part ? reinterpret_cast<float2*>(part + (size_t)wgs * splits * kPaRows * HD) : nullptr;
     hipLaunchKernelGGL(attention_rows_mfma_kernel<HD>, dim3((unsigned)nkv, (unsigned)tiles, (unsigned)splits),
