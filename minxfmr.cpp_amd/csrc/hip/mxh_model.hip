@@ -94,8 +94,7 @@ struct mxh_model {
     uint16_t *pf_h16 = nullptr, *pf_l16 = nullptr, *pf_sh = nullptr, *pf_sl = nullptr;
     float* pf_rscale = nullptr;
     bool bf16_prefill = false;  // every prefill GEMM in the split-bf16 form
-    float* pf_part = nullptr;                        // split-K partial tiles
-    size_t pf_part_floats = 0;
+    size_t pf_part_floats = 0;  // split-K partial tiles of a bf16 GEMM, in the library stream's workspace
 };
 
 namespace {
@@ -283,7 +282,7 @@ int free_model(mxh_model* m) {
         drop_graph(*g);
     void* bufs[] = {m->blob, m->out_copy, m->kv, m->rope_cs, m->x, m->xn, m->qkv, m->att, m->gu, m->h, m->logits, m->part,
                     m->trace, m->tokens, m->pos, m->red_val, m->red_idx,
-                    m->pf_x, m->pf_qkv, m->pf_q, m->pf_att, m->pf_gu, m->pf_a, m->pf_a_lo, m->pf_part,
+                    m->pf_x, m->pf_qkv, m->pf_q, m->pf_att, m->pf_gu, m->pf_a, m->pf_a_lo,
                     m->pf_h16, m->pf_l16, m->pf_sh, m->pf_sl, m->pf_rscale, m->sprm, m->scand, m->eprm, m->esup,
                     m->ecnt};
     for (void* b : bufs)
@@ -761,8 +760,9 @@ int ensure_prefill_buffers(mxh_model* m) {
     if (!rc) rc = dalloc(&m->pf_sl, (size_t)rows * (widest / 32));
     if (!rc) rc = dalloc(&m->pf_rscale, (size_t)rows);
     // split-K partials: up to 4 splits of the narrower outputs (x, q|k|v)
-    m->pf_part_floats = 4 * (size_t)rows * std::max((size_t)c.n_embd, qd + 2 * kvd);
-    if (!rc) rc = dalloc(&m->pf_part, m->pf_part_floats);
+    size_t shared = 0;
+    (void)gemm_partials(&shared);
+    m->pf_part_floats = std::min(4 * (size_t)rows * std::max((size_t)c.n_embd, qd + 2 * kvd), shared / sizeof(float));
     if (!rc) m->pf_rows = rows;
     return rc;
 }
@@ -779,8 +779,10 @@ int gemm(mxh_model* m, const DevW& w, int lda, float* out, int ldo, const float*
     if (f16_gemm(m, w))
         return gemm_q_f16_run(w.type, m->pf_h16, m->pf_l16, lda, m->pf_sh, m->pf_sl, lda / 32, m->pf_rscale, w.p,
                                 out, ldo, res, rows, (int)w.rows, (int)w.cols, m->form, Workspace::kStream, st);
+    size_t shared = 0;
+    float* part = reinterpret_cast<float*>(gemm_partials(&shared));
     return gemm_bf16_run(w.type, m->pf_a, m->pf_a_lo, lda, w.p, out, ldo, res, rows, (int)w.rows, (int)w.cols,
-                         m->form, m->pf_part, m->pf_part_floats, st);
+                         m->form, part, m->pf_part_floats, st);
 }
 
 // GEMM inputs from rows of x (normed with nw when given) in the forms the
