@@ -1729,6 +1729,13 @@ int gemv_run(int type, const GemvArgs& a, int mode, hipStream_t st) {
     return MXH_ERR_UNSUPPORTED;
 }
 
+// Long F16 and F32 rows go two rows of x at a time; where two weight rows a
+// wave then leave CUs idle, one a wave.  us for 3 / 5 rows of x at 256 x 14336,
+// loop of GEMVs, two a wave, one a wave: F16 26.5 37.7 22.6 / 46.3 56.0 31.2,
+// F32 77 90 51 / 126 144 70; at 512 x 4096 two a wave are as fast or faster
+// (F16, 2 rows: 5.7 against 6.6).
+static bool one_row_a_wave(int n, int k) { return k > 4096 && n <= kRowsWaves * device_cus(); }
+
 int gemv_rows_run(int type, const void* w, const float* x, float* y, int m, int n, int k, int form, hipStream_t st) {
     if (k % 32 || k > kGemvMaxK || n <= 0 || m <= 0) return MXH_ERR_ARG;
     const uint8_t* wb = (const uint8_t*)w;
@@ -1745,8 +1752,12 @@ int gemv_rows_run(int type, const void* w, const float* x, float* y, int m, int 
     case MXH_Q8_0: return rows_launch<Q80, 2>(wb, x, y, m, n, k, form, st);
     case MXH_Q8_0_TILED: return rows_launch<Q80T, 2>(wb, x, y, m, n, k, form, st);
     case MXH_Q5_0: return rows_launch<Q50, 2>(wb, x, y, m, n, k, form, st);
-    case MXH_F16: return rows_launch<F16W, 2>(wb, x, y, m, n, k, form, st);
-    case MXH_F32: return rows_launch<F32W, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_F16:
+        return one_row_a_wave(n, k) ? rows_launch<F16W, 1>(wb, x, y, m, n, k, form, st)
+                                 : rows_launch<F16W, 2>(wb, x, y, m, n, k, form, st);
+    case MXH_F32:
+        return one_row_a_wave(n, k) ? rows_launch<F32W, 1>(wb, x, y, m, n, k, form, st)
+                                 : rows_launch<F32W, 2>(wb, x, y, m, n, k, form, st);
     }
     return MXH_ERR_UNSUPPORTED;
 }

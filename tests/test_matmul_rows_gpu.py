@@ -52,3 +52,10 @@ def test_matmul_rows_equal_gemvs(mxh, name, m, n, k, tiled):
     assert np.all(got[m * n:] == 7.0)
     for b in (dw, dx, out, ref):
         b.close()
+
+
+# long fp32 and fp16 rows: one weight row a wave up to eight per CU, two above
+@pytest.mark.parametrize("m,n,k", [(2, 2048, 4128), (3, 2049, 4128), (5, 257, 4096), (9, 300, 5024), (5, 7, 14336)])
+@pytest.mark.parametrize("name", ["F16", "F32"])
+def test_long_float_rows_equal_gemvs(mxh, name, m, n, k):
+    test_matmul_rows_equal_gemvs(mxh, name, m, n, k, False)
