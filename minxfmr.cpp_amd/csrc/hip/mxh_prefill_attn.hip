@@ -18,13 +18,14 @@
 //   S^T = K Q^T      v_mfma_f32_32x32x16_f16; q is pre-scaled by
 //                    log2(e) / sqrt(hd) and split into fp16 hi + lo (about
 //                    22 significant bits); K is exact (the cache is fp16)
-//   O^T += V^T P^T   P = 2^(S - ref + 6) split into fp16 hi + lo; V exact
+//   O^T += V^T P^T   P = 64 2^(S - ref) split into fp16 hi + lo; V exact
 //
 // ref is the row's largest score when it was last set: it moves (and the sums
 // are rescaled, all by one rounded factor) only where a score exceeds it by
-// more than 8, which is rare.  The 2^6 keeps the low halves of small probabilities out of the
-// fp16 subnormals (2 queries at 7000 against float64: 9.5e-7 without, 5.6e-7
-// with), and P stays below 2^14.
+// more than 8, which is rare.  The factor 64 keeps the low halves of small
+// probabilities out of the fp16 subnormals, and P stays at most 2^14.  It is
+// multiplied, not added to the exponent: 6 + (S - ref) would be rounded at the
+// magnitude of 6 (rms error of near-equal probabilities 1.3e-7, 7.4e-8 so).
 //
 // Lane l owns query l % 32 in both products (accumulator register i of lane l
 // is row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32), so the softmax
@@ -67,7 +68,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPaRows = 64;        // query rows per workgroup
-constexpr float kPaBias = 6.f, kPaSlack = 8.f;  // P at most 2^(bias + slack)
+constexpr float kPaScale = 64.f, kPaSlack = 8.f;  // P at most scale 2^slack
 
 constexpr int kPaKeys = 64;        // keys per stage
 constexpr int kPaThreads = 256;
@@ -252,11 +253,11 @@ __global__ __launch_bounds__(kPaThreads, 2) void attention_rows_mfma_kernel(
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
             }
-            const float bias = mref == -INFINITY ? 0.f : kPaBias - mref;
+            const float ref0 = mref == -INFINITY ? 0.f : mref;
             float p[16], ps[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                p[v] = __builtin_amdgcn_exp2f(s[v] + bias);
+                p[v] = kPaScale * __builtin_amdgcn_exp2f(s[v] - ref0);
                 ps[v & 3] += p[v];
             }
             lrun += (ps[0] + ps[1]) + (ps[2] + ps[3]);

@@ -68,3 +68,33 @@ def test_attention_probabilities_are_unbiased(mxh, nh, nkv, hd, p0, m):
     assert abs(err.mean()) <= 2.0 ** -25, f"mean error {err.mean():.3g}"
     for b in (dq, dk, dv, att):
         b.close()
+
+
+def test_attention_near_equal_probabilities(mxh):
+    """The rms error of single probabilities of nearly equal scores.  Scores are
+    exact (one fp16 q value times one K value), V picks one key a dim.  exp2's
+    last place, the split and the quotient leave 7.4e-8; an exponent rounded at
+    a magnitude of 4 to 8 adds 2^-21 / sqrt(12) ln 2 = 9.5e-8: 1.2e-7 and more.
+    """
+    nh, nkv, hd, n = 8, 2, 128, 100
+    qscale = np.float32(1.0) / np.sqrt(np.float32(hd)) * np.float32(1.4426950408889634)
+    errs = []
+    for seed in range(20):
+        rng = np.random.default_rng(seed)
+        c = np.float32(np.float16(1.0 + rng.random()))  # the scaled q the kernel is to see, exact in fp16
+        near = np.float32(c / qscale)
+        q0 = next(x for x in (near, np.nextafter(near, np.float32(9)), np.nextafter(near, np.float32(-9))) if x * qscale == c)
+        q, kc, vc = np.zeros((1, nh, hd), np.float32), np.zeros((n, nkv, hd), np.float16), np.zeros((n, nkv, hd), np.float16)
+        q[0, :, 5] = q0
+        kc[:, :, 5] = 0.1 * rng.standard_normal((n, nkv))
+        vc[np.arange(n), :, np.arange(n)] = 1
+        dq, dk, dv = (mxhip.DeviceBuffer.from_array(a.reshape(len(a), -1)) for a in (q, kc, vc))
+        att = mxhip.DeviceBuffer(4 * nh * hd)
+        mxhip.attention_prefill(dq, dk, dv, att, n - 1, 1, nh, nkv, hd)
+        got = att.download(np.float32, nh * hd).reshape(nh, hd)[:, :n].astype(np.float64)
+        p = 2.0 ** (float(c) * kc[:, :, 5].astype(np.float64))
+        errs.append(got / np.repeat((p / p.sum(0)).T, nh // nkv, axis=0) - 1)
+        for b in (dq, dk, dv, att):
+            b.close()
+    rms = float(np.sqrt(np.mean(np.square(errs))))
+    assert rms <= 1e-7, f"rms error {rms:.3g}"
