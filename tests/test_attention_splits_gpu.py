@@ -98,3 +98,26 @@ def test_attention_near_equal_probabilities(mxh):
             b.close()
     rms = float(np.sqrt(np.mean(np.square(errs))))
     assert rms <= 1e-7, f"rms error {rms:.3g}"
+
+
+@pytest.mark.parametrize("nh,nkv,hd,p0,m", [(8, 2, 128, 0, 300), (8, 8, 64, 500, 100), (4, 1, 32, 3000, 64)],
+                         ids=["d128", "d64", "split"])
+def test_attention_error_is_that_of_22_bits(mxh, nh, nkv, hd, p0, m):
+    """2-norm error against float64 at ordinary scores.  q as fp16 hi + lo is
+    off by 2^-23 of itself at most, a score (in base 2, |s| about 1.4) by about
+    as much of its terms: 2e-7 to 5e-7 of the outputs with the sums.  One q in
+    some thousand with halves that do not belong together (2^-12 off) made it
+    4e-6 to 1.2e-5.  2^-20 (9.5e-7) lies between.
+    """
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((m, nh * hd)).astype(np.float32)
+    kc, vc = (rng.standard_normal((p0 + m, nkv * hd)).astype(np.float16) for _ in range(2))
+    dq, dk, dv = (mxhip.DeviceBuffer.from_array(a) for a in (q, kc, vc))
+    att = mxhip.DeviceBuffer(4 * m * nh * hd)
+    mxhip.attention_prefill(dq, dk, dv, att, p0, m, nh, nkv, hd)
+    got = att.download(np.float32, m * nh * hd).reshape(m, nh * hd).astype(np.float64)
+    want = reference(q, kc, vc, p0, m, nh, nkv, hd)
+    rel = float(np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert rel <= 2.0 ** -20, f"relative error {rel:.3g}"
+    for b in (dq, dk, dv, att):
+        b.close()
