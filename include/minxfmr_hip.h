@@ -302,7 +302,9 @@ int mxh_model_set_logit_edits(mxh_model *m, const int *suppress, int n_suppress,
 
 /* One sampling decision over n device-resident logits with the rules of
  * mxh_model_set_sampling, using draw number `draw` of the stream; the token
- * id is written to *token (host).  For tests and per-op callers. */
+ * id is written to *token (host).  top_k up to 64 takes n up to 2^24 / top_k
+ * ids (top_k to the next power of two; 2^23 at most), above it any n.  For
+ * tests and per-op callers. */
 int mxh_sample(const float *logits, int n, int top_k, double temperature, double top_p, double min_p, uint64_t seed,
                uint64_t draw, int *token);
 

@@ -79,7 +79,7 @@ struct mxh_model {
     bool sampling = false;
     int top_k = 1;
     SampleParams* sprm = nullptr;  // device copy, draw counter included
-    uint64_t* scand = nullptr;     // pass-1 candidates
+    uint64_t* scand = nullptr;     // group maxima
     // logit edits before the choice (mxh_model_set_logit_edits)
     bool edits = false;
     EditParams* eprm = nullptr;  // device copy
@@ -89,7 +89,7 @@ struct mxh_model {
     int pf_rows = 0;
     float *pf_x = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_att = nullptr, *pf_gu = nullptr;
     uint16_t *pf_a = nullptr, *pf_a_lo = nullptr;  // GEMM input as split bf16 (hi, lo)
-    // GEMM input of the Q4_K fp16 kernel: fp16 hi / lo of a * 2^e per row,
+    // GEMM input of the exact-weight kernel: fp16 hi / lo of a * 2^e per row,
     // split sub-block sums, 2^-e per row
     uint16_t *pf_h16 = nullptr, *pf_l16 = nullptr, *pf_sh = nullptr, *pf_sl = nullptr;
     float* pf_rscale = nullptr;

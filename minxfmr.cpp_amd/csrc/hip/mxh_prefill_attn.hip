@@ -44,7 +44,7 @@
 // Bound: a block's 32 MFMAs (1,024 cycles at head dim 128) and its softmax
 // (165 vector instructions, about 850 cycles) follow each other in a wave, and
 // the two waves of a SIMD keep in step, so their times add up (counters at 512
-// queries at 7680: matrix cores busy 43%, vector ALU 50%).  So the vector work
+// queries at 7680: matrix cores busy 48%, vector ALU 45%).  So the vector work
 // was cut: the reference that seldom moves, one-instruction splits, loads
 // without masks.  228 -> 156 us there; the first product one block ahead needs
 // more registers than there are (spills, 258 us), wave priorities change

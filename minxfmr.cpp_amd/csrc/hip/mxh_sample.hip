@@ -416,7 +416,8 @@ __global__ __launch_bounds__(kThreads) void choose_topk_kernel(const float* __re
 size_t sample_scratch_keys(int n) { return ((size_t)group_count(n) + 1) / 2; }
 
 // Vocabularies taken: any for top_k above 64, else up to 4096 times 4096 /
-// top_k (to the next power of two) ids, 8M at most.
+// top_k (to the next power of two) ids, 8M at most.  The kernels have no such
+// limit; it is what the entry point and the models have always refused.
 int sample_launch(const float* logits, int n, SampleParams* prm, const SampleParams* call, int top_k, uint64_t* cand,
                   int* out, int* tokens, int* pos, hipStream_t st) {
     if (n <= 0 || top_k < 1 || top_k > kSampleTopKMax || top_k > n) return MXH_ERR_ARG;

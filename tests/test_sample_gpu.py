@@ -3,8 +3,7 @@
 
 The oracle (oracle/mxo.c: mxo_sample) restates minxfmr.cpp:2091-2171 with a
 seeded splitmix64 draw; the device sampler must pick the same id for the
-same logits and the same draw number.  top_k up to 64 takes the two-pass
-form, 65..4096 the one-workgroup radix-select form.
+same logits and the same draw number, for every top_k it takes (1..4096).
 """
 from __future__ import annotations
 
@@ -45,9 +44,8 @@ def test_sample_matches_oracle_on_fixed_logits(mxh, n, k, t, p, mp):
 @pytest.mark.parametrize("k,t,p,mp", [(8, 0.8, 1.0, 0.0), (64, 1.0, 1.0, 0.1), (40, 0.7, 0.95, 0.05),
                                      (500, 1.0, 1.0, 0.0)])
 def test_sample_top_values_in_one_slice(mxh, k, t, p, mp):
-    """The largest logits sit at consecutive ids, inside one first-pass
-    slice (and straddling the next): the second pass must still see all of
-    them, whichever lists it keeps."""
+    """The largest logits sit at consecutive ids, side by side in their groups:
+    the choice must still see all of them, whichever groups it reads again."""
     n = 151936
     rng = np.random.default_rng(k)
     logits = (rng.standard_normal(n) * 0.5).astype(np.float32)
@@ -78,7 +76,7 @@ from test_model_gpu import TINY, build  # noqa: E402
                                         ("q4k-qknorm", 8, 40)])
 def test_model_sampling_matches_oracle(mxh, tmp_path, name, k, n_ctx):
     """Seeded top-k=8, T=0.8 decoding (the BASELINE Llama-3 workload's
-    sampler) of a tiny model, and top-k 100 (the radix-select form, inside
+    sampler) of a tiny model, and top-k 100 (inside
     the captured decode graph): a reset replays the same stream; graph
     replay equals eager launches; every id is the oracle sampler's choice
     over the device's own logits at that step (a greedy twin model fed the
