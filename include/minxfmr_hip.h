@@ -180,7 +180,7 @@ int mxh_gemm_q_f16_noalloc(int type, const float *a, int64_t m, const void *w, i
  * keys among workgroups, their parts going through the library stream's shared
  * static memory (see mxh_gemm_q_f16); recorded in a graph (the library stream
  * capturing) a call does not split, so its replays use the caller's buffers
- * alone and may overlap anything. */
+ * alone and may overlap anything (the outputs agree to fp32 rounding). */
 int mxh_attention_prefill(const float *q, const void *kc, const void *vc, float *att, int p0, int m, int nh, int nkv,
                           int hd);
 

@@ -1003,10 +1003,13 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
     const size_t rb = row_bytes(MXH_Q6_K, 256 * (int64_t)a.row_blocks);  // of a regrouped row
     // regrouped rows go through the slab in equal pieces, whole tiles of rows,
     // each under the plan for what it launches (2 x 30000 x 11008 under a plan
-    // for all rows: seven launches of a seventh of the chip)
+    // for all rows: seven launches of a seventh of the chip) - but under one for
+    // all rows where the rows have a tiled order too, whose results are these
     const int slab_rows = regroup ? (int)(kSlabBytes / rb / 256 * 256) : n;
     const int pieces = (n - 1) / slab_rows + 1;
     const int step = pieces > 1 ? ((n - 1) / pieces + 256) / 256 * 256 : n;
+    GemmPlan p = gemm_plan(f, m, n, k, device_cus(), kPartBytes);
+    const bool per_piece = pieces > 1 && tiled_type(type, k) == type;
     for (int n0 = 0; n0 < n; n0 += step) {
         const int nn = std::min(step, n - n0);
         const uint8_t* src = static_cast<const uint8_t*>(w) + (size_t)n0 * in_rb;
@@ -1017,7 +1020,7 @@ int gemm_q_f16_run(int type, const uint16_t* a_hi, const uint16_t* a_lo, int lda
                                g_slab_ptr, nn, k, a.row_blocks);
             a.w = g_slab_ptr;
         }
-        const GemmPlan p = gemm_plan(f, m, nn, k, device_cus(), kPartBytes);
+        if (per_piece) p = gemm_plan(f, m, nn, k, device_cus(), kPartBytes);
         a.blocks = p.blocks, a.splits = p.splits;
         a.n = nn;
         a.out = out + n0;

@@ -25,22 +25,22 @@ struct GemmPlan {
 // the step's time lying between what it takes on a nearly idle chip and on a
 // full one (ns, measured per format and tile at K = 4096 .. 14336, where the
 // estimate is within 10% of the measured time of the shapes tried); 7.5 us is
-// what a work item takes to start, fill its stages and store its outputs.  The
-// rows in GGUF order were fitted from K = 1024 on, with that time per tile too
-// (rms 5 to 9%).
+// what a work item takes to start, fill its stages and store its outputs.  Q5_0
+// was fitted from K = 1024 on, with that time per tile too (rms 5 to 9%).  A
+// type's two orders, GGUF and tiled, share their costs: the split of K is part
+// of the results, and these are the same bits through either.
 inline GemmPlan gemm_plan(GemmFmt fmt, int m, int n, int k, int cus, size_t part_bytes) {
     struct Cost {
         float idle, full, item = 7500.f;
     };
-    static const Cost cost[6][GT_COUNT] = {
+    static const Cost cost[5][GT_COUNT] = {
         {{1420.f, 2130.f}, {830.f, 1160.f}, {800.f, 1110.f}, {490.f, 650.f}},       // Q4_K
         {{1680.f, 2280.f}, {980.f, 1270.f}, {950.f, 1220.f}, {650.f, 830.f}},       // Q5_K
         {{1720.f, 2300.f}, {980.f, 1180.f}, {950.f, 1200.f}, {600.f, 830.f}},       // Q8_0
         {{1e6f, 1e6f}, {1430.f, 1730.f}, {1560.f, 1830.f}, {1000.f, 1130.f}},       // Q6_K
-        {{1880.f, 2180.f, 8000.f}, {960.f, 1210.f, 4300.f}, {1070.f, 1280.f, 4400.f}, {830.f, 990.f, 2500.f}},  // Q8_0 in GGUF order
         {{2460.f, 2470.f, 9100.f}, {1350.f, 1350.f, 5300.f}, {1250.f, 1280.f, 5500.f}, {1140.f, 780.f, 2000.f}}};  // Q5_0
     static const int bm[GT_COUNT] = {128, 128, 64, 32}, bn[GT_COUNT] = {256, 128, 256, 256};
-    static const int cls_of[] = {0, 0, 1, 1, 4, 2, 5, 3};  // by GemmFmt
+    static const int cls_of[] = {0, 0, 1, 1, 2, 2, 4, 3};  // by GemmFmt
     const int cls = cls_of[fmt], nblk = k / 256;
     GemmPlan best{GT_128x256, nblk, 1};
     double best_cost = 1e30;

@@ -111,3 +111,19 @@ def test_q6k_more_than_one_slab(mxh, m):
         alone = gemm(mxo.Q6_K, a, dw.ptr + n0 * rb, nn, k, res=np.ascontiguousarray(res[:, n0:n0 + nn]), ldo=nn)
         assert np.array_equal(alone.view(np.uint32), np.ascontiguousarray(got[:, n0:n0 + nn]).view(np.uint32))
     dw.close()
+
+
+def test_q6k_orders_give_the_same_bits_beyond_a_slab(mxh):
+    """Rows that have a tiled order too (k a multiple of 2048): the pieces keep
+    the K split of the call over all rows, which is that of the tiled rows."""
+    m, n, k = 3, 10240, 14336
+    rng = np.random.default_rng(9)
+    raw = rng.integers(0, 256, (64, k // 256, 210), dtype=np.uint8)
+    raw[:, :, 208:210] = (rng.standard_normal((64, k // 256, 1)) * 0.01).astype(np.float16).view(np.uint8)
+    dw = mxhip.DeviceBuffer.from_array(np.tile(raw.reshape(64, -1), (n // 64, 1)))
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    gguf = gemm(mxo.Q6_K, a, dw.ptr, n, k)
+    t = mxhip.tile_rows(mxo.Q6_K, dw, n, k)
+    assert t != mxo.Q6_K
+    assert np.array_equal(gguf.view(np.uint32), gemm(t, a, dw.ptr, n, k).view(np.uint32))
+    dw.close()

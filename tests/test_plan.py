@@ -76,3 +76,12 @@ def test_plans_follow_the_cu_count(lib):
     # 8 workgroups over 121 stages
     wide, narrow = attn(lib, 128, 8, 121, 256)[1], attn(lib, 128, 8, 121, 32)[1]
     assert wide > 2 * narrow >= 2
+
+
+def test_both_orders_of_a_type_have_one_plan(lib):
+    # (GGUF order, tiled) of Q4_K, Q5_K, Q8_0: the same K split, so the same bits
+    for gguf, tiled in ((0, 1), (2, 3), (4, 5)):
+        for m in (1, 19, 64, 200, 512):
+            for n in (256, 1030, 4096, 28672):
+                for k in (256, 512, 4096, 14336):
+                    assert gemm(lib, gguf, m, n, k, 256) == gemm(lib, tiled, m, n, k, 256)
